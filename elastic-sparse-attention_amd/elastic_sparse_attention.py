@@ -890,7 +890,7 @@ def elastic_attention_bwd_rows(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
     _check_qkv(q, k, v)
     B, H, Lq, D = q.shape
     q, k, v = _prep(q, 4), _prep(k, 4), _prep(v, 4)
-    dout = dout.to(q.dtype)
+    dout = _prep(dout.to(q.dtype), 4)
     lse = lse.contiguous()
     dq = torch.empty(B, H, Lq, D, dtype=q.dtype, device=q.device)
     dk = torch.empty_like(k, memory_format=torch.contiguous_format)
@@ -928,7 +928,7 @@ def sparse_attention_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: t
     _check_qkv(q, k, v)
     B, H, Lq, D = q.shape
     q, k, v = _prep(q, 4), _prep(k, 4), _prep(v, 4)
-    dout = dout.to(q.dtype)
+    dout = _prep(dout.to(q.dtype), 4)
     idx, msk = _index_arrays(sparse_indices, sparse_mask)
     dq = torch.empty(B, H, Lq, D, dtype=q.dtype, device=q.device)
     dk = torch.empty_like(k, memory_format=torch.contiguous_format)
