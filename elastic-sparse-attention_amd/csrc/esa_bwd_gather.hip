@@ -29,9 +29,16 @@
 //                     coefficient * q row and dV = sum of coefficient * dO
 //                     row over the key's entries, in entry order.
 //
-// Every gradient element is summed by one wave in a fixed order, so two
-// runs agree bit for bit.  The index lists do not depend on the batch, so
+// The row and key-major passes have a cooperative-row form each
+// (rows_coop_kernel, kv_coop_kernel, below), taken for 16-byte aligned rows;
+// the per-lane forms above serve the rest.
+//
+// Every gradient element is summed by one wave (a long key segment by one wave
+// per window, the windows in order) in a fixed order, so two runs agree bit
+// for bit.  The index lists do not depend on the batch, so
 // the sort serves every batch element.
+#include <type_traits>
+
 #include "esa_gather.hpp"
 
 namespace esa {
@@ -231,6 +238,362 @@ __global__ __launch_bounds__(256) void bwd_kv_kernel(GatherBwdArgs A) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Cooperative-row forms of the two passes (rows_coop_kernel, kv_coop_kernel):
+// LPK lanes read each row, 16 bytes a lane, so a load instruction covers KPI =
+// 64 / LPK whole rows (bwd_rows_kernel walks a K row per lane, 64 cache lines
+// an instruction, and reads K twice).  Taken when coop_applies: 16-byte
+// aligned rows and spans that 32-bit buffer offsets reach.  Loads go through
+// buffer resources: a masked entry, a slot past a key's entries or a lane past
+// head_dim gets an offset past num_records and reads zeros without a fetch, so
+// a row that is not listed never meets the sums (no 0 * Inf).  Kernel times,
+// per-lane forms against these: bf16 B=2 H=8 L=4096 D=128 (2.1 GB of rows in
+// each pass) row pass 520 -> 203 us, key pass 787 -> 155 us (13.9 TB/s);
+// float32 B=2 H=8 L=4096 D=64 467 -> 154 and 564 -> 106 us; bf16 D=96 H=16/4
+// L=5001 496 -> 231 and 1036 -> 236 us.
+
+constexpr uint32_t kOffNone = 0x80000000u;   // an entry's row offset: none
+constexpr uint32_t kLaneNone = 0x7FFFF000u;  // a lane's offset within a row: past head_dim
+// spans stay below both offsets
+constexpr int64_t kMaxSpan = (int64_t(1) << 31) - 8192;
+
+__device__ __forceinline__ u32x4 load16(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
+  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
+}
+
+// v of lane `src` (0 .. 63)
+__device__ __forceinline__ uint32_t from_lane(uint32_t v, int src) {
+  return (uint32_t)__builtin_amdgcn_ds_bpermute(4 * src, (int)v);
+}
+__device__ __forceinline__ float from_lane(float v, int src) {
+  return __uint_as_float(from_lane(__float_as_uint(v), src));
+}
+
+template <Elem E>
+__device__ __forceinline__ float dot16(const u32x4& a, const u32x4& b) {
+  float acc = 0.f;
+#pragma unroll
+  for (int e = 0; e < ElemT<E>::kPerChunk; ++e) acc += ElemT<E>::chunk(a, e) * ElemT<E>::chunk(b, e);
+  return acc;
+}
+
+// sum over the lanes l, l + LPK, l + 2 LPK, ... (a row slot each)
+template <int LPK>
+__device__ __forceinline__ float slot_sum(float v) {
+#pragma unroll
+  for (int off = LPK; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+// One wave per (batch, head, query row): dQ and the row's (lse, delta).  A
+// chunk's K and V rows (up to 64 entries) are all in flight before the first
+// score, K stays in registers for dQ, and each lane forms one entry's dS.
+// Bound by the L2 row gathers (2 w rows a query row).
+template <Elem E, int LPK, bool PATTERN>
+__global__ __launch_bounds__(256, 2) void rows_coop_kernel(GatherBwdArgs A) {
+  using T = typename ElemT<E>::T;
+  constexpr int EPL = ElemT<E>::kPerChunk;
+  constexpr int KPI = 64 / LPK;
+  constexpr int SK = 16 * KPI < 64 ? 16 * KPI : 64;  // entries per chunk
+  constexpr int NI = SK / KPI;
+  __shared__ float s_all[4][64];
+  __shared__ float dp_all[4][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  // XCD x (blockIdx % 8) takes a contiguous range of rows, so it reads few
+  // heads' K and V at a time
+  const int blk = (int)(blockIdx.x & 7) * A.rows_per_xcd + (int)(blockIdx.x >> 3);
+  const int hr = blk * 4 + wave;
+  const int b = blockIdx.y;
+  if (hr >= A.H * A.q_len) return;  // whole wave leaves; no block-level barrier below
+  const int h = hr / A.q_len, r = hr % A.q_len;
+  const int kvh = h / A.groups;
+  const int gk = lane / LPK, ln = lane % LPK;
+  const bool act = ln * EPL < A.D;
+  const uint32_t lofs = act ? 16u * (uint32_t)ln : kLaneNone;
+  float* sl = s_all[wave];
+  float* dpl = dp_all[wave];
+
+  u32x4 q16 = {0u, 0u, 0u, 0u}, g16 = q16, o16 = q16;
+  if (act) {
+    q16 = *(const u32x4*)((const T*)A.q + (int64_t)b * A.qsb + (int64_t)h * A.qsh +
+                          (int64_t)r * A.qss + EPL * ln);
+    g16 = *(const u32x4*)((const T*)A.dout + (int64_t)b * A.dosb + (int64_t)h * A.dosh +
+                          (int64_t)r * A.doss + EPL * ln);
+    o16 = *(const u32x4*)((const T*)A.o + (int64_t)b * A.osb + (int64_t)h * A.osh +
+                          (int64_t)r * A.oss + EPL * ln);
+  }
+  RowEntries row;
+  row.init<PATTERN>(A.src, h, r);
+  const float lse = A.lse[(int64_t)b * A.lsb + (int64_t)h * A.lsh + r];
+  const float delta = group_sum<LPK>(dot16<E>(g16, o16));
+
+  const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)((const T*)A.k + (int64_t)b * A.ksb + (int64_t)kvh * A.ksh), (short)0, A.k_span,
+      0x00020000);
+  const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)((const T*)A.v + (int64_t)b * A.vsb + (int64_t)kvh * A.vsh), (short)0, A.v_span,
+      0x00020000);
+  const int w = A.src.w;
+  const uint32_t kst = (uint32_t)A.kss * sizeof(T), vst = (uint32_t)A.vss * sizeof(T);
+
+  float acc[EPL];
+#pragma unroll
+  for (int e = 0; e < EPL; ++e) acc[e] = 0.f;
+  bool dead = false;
+  for (int c0 = 0; c0 < w; c0 += SK) {
+    const int j = c0 + lane;
+    bool valid = false;
+    int64_t key = 0;
+    if (lane < SK && j < w) row.entry<PATTERN>(A.src, h, r, j, valid, key);
+    const bool live = valid && key >= 0 && key < A.kv_len && !row.bad_pos;
+    dead |= lane < SK && j < w && !live;
+    const uint32_t ko = live ? (uint32_t)key * kst : kOffNone;
+    const uint32_t vo = live ? (uint32_t)key * vst : kOffNone;
+    u32x4 kd[NI], vd[NI];
+#pragma unroll
+    for (int t = 0; t < NI; ++t) {
+      kd[t] = load16(rk, from_lane(ko, KPI * t + gk) + lofs);
+      vd[t] = load16(rv, from_lane(vo, KPI * t + gk) + lofs);
+    }
+#pragma unroll
+    for (int t = 0; t < NI; ++t) {
+      const float s = group_sum<LPK>(dot16<E>(q16, kd[t]));
+      const float dp = group_sum<LPK>(dot16<E>(g16, vd[t]));
+      if (ln == 0) {
+        sl[KPI * t + gk] = s;
+        dpl[KPI * t + gk] = dp;
+      }
+    }
+    wave_sync_lds();
+    float dsc = 0.f;
+    if (live) {
+      const float p = expf(sl[lane] * A.sm_scale - lse);
+      const float keep = drop_factor(A.drop, b, h, r, j, A.H, A.q_len, w);
+      dsc = p * (keep * dpl[lane] - delta) * A.sm_scale;
+    }
+    wave_sync_lds();
+    if (lane < SK) sl[lane] = dsc;
+    wave_sync_lds();
+#pragma unroll
+    for (int t = 0; t < NI; ++t) {
+      const float g = sl[KPI * t + gk];
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) acc[e] += g * ElemT<E>::chunk(kd[t], e);
+    }
+    wave_sync_lds();
+  }
+#pragma unroll
+  for (int e = 0; e < EPL; ++e) acc[e] = slot_sum<LPK>(acc[e]);
+  // (as bwd_rows_kernel: NaN for an entry not attended when delta is not finite)
+  const bool all_nan = row.bad_pos || (__builtin_amdgcn_ballot_w64(dead) != 0 &&
+                                       !__builtin_isfinite(delta));
+  if (all_nan) {
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) acc[e] = __builtin_nanf("");
+  }
+  if (gk == 0 && act)
+    *(u32x4*)((T*)A.dq + (int64_t)b * A.dqsb + (int64_t)h * A.dqsh + (int64_t)r * A.dqss +
+              EPL * ln) = ElemT<E>::pack_chunk(acc);
+  if (lane == 0) A.ld2[(int64_t)b * A.H * A.q_len + hr] = make_float2(lse, delta);
+}
+
+// dK and dV of one (batch, kv head, key) over sorted positions [i0, i1) of
+// its entries, in entry order: each entry's p and dS are formed again from
+// its q and dO rows and the row's (lse, delta), so no coefficient per entry
+// passes through memory.  A lane decodes one of 64 entries (row offsets, lse,
+// delta); U loads of KPI rows each of q and dO are in flight per step; the
+// exponential of the step's U * KPI entries is formed once, lane ln of a row
+// taking entry ln % U, and handed to the row's lanes by quad broadcasts.
+template <Elem E, int LPK>
+struct KvAcc {
+  static constexpr int EPL = ElemT<E>::kPerChunk;
+  static constexpr int KPI = 64 / LPK;
+  static constexpr int U = 4;
+  float dk[EPL], dv[EPL];
+
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) dk[e] = dv[e] = 0.f;
+  }
+
+  __device__ __forceinline__ void run(const GatherBwdArgs& A, int b, const u32x4& k16,
+                                      const u32x4& v16, int i0, int i1, int lane) {
+    using T = typename ElemT<E>::T;
+    const int gk = lane / LPK, ln = lane % LPK;
+    const uint32_t lofs = ln * EPL < A.D ? 16u * (uint32_t)ln : kLaneNone;
+    const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)((const T*)A.q + (int64_t)b * A.qsb), (short)0, A.q_span, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)((const T*)A.dout + (int64_t)b * A.dosb), (short)0, A.do_span, 0x00020000);
+    const float2* ld2 = A.ld2 + (int64_t)b * A.H * A.q_len;
+    const int w = A.src.w;
+    for (int ib = i0; ib < i1; ib += 64) {
+      uint32_t qo = kOffNone, go = kOffNone;
+      float lse = 0.f, delta = 0.f, keep = 1.f;
+      if (ib + lane < i1) {
+        const uint32_t e = A.vals_out[ib + lane];
+        const uint32_t hr = fast_div(e, A.div_w);
+        const uint32_t h = fast_div(hr, A.div_q);
+        const uint32_t r = hr - h * (uint32_t)A.q_len;
+        qo = (h * (uint32_t)A.qsh + r * (uint32_t)A.qss) * (uint32_t)sizeof(T);
+        go = (h * (uint32_t)A.dosh + r * (uint32_t)A.doss) * (uint32_t)sizeof(T);
+        const float2 x = ld2[hr];
+        lse = x.x;
+        delta = x.y;
+        if (A.drop.p > 0.f)
+          keep = drop_factor(A.drop, b, (int)h, (int)r, (int)(e - hr * (uint32_t)w), A.H, A.q_len,
+                             w);
+      }
+      const int n = min(i1 - ib, 64);
+      for (int t0 = 0; t0 < n; t0 += U * KPI) {
+        u32x4 qd[U], gd[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int src = t0 + u * KPI + gk;
+          qd[u] = load16(rq, from_lane(qo, src) + lofs);
+          gd[u] = load16(rg, from_lane(go, src) + lofs);
+        }
+        // this lane's entry of the step's four: u = ln % 4
+        const int mine = t0 + (ln & 3) * KPI + gk;
+        const float lse_m = from_lane(lse, mine), delta_m = from_lane(delta, mine);
+        float keep_m = 1.f;
+        if (A.drop.p > 0.f) keep_m = from_lane(keep, mine);
+        float s = 0.f, dp = 0.f;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const float su = group_sum<LPK>(dot16<E>(k16, qd[u]));
+          const float du = group_sum<LPK>(dot16<E>(v16, gd[u]));
+          s = (ln & 3) == u ? su : s;
+          dp = (ln & 3) == u ? du : dp;
+        }
+        // (a slot past the entries: zero rows with coefficient 0, also where
+        // the key's own row is not finite)
+        const bool in = mine < n;
+        const float p = expf(s * A.sm_scale - lse_m);
+        const float pc = in ? keep_m * p : 0.f;
+        const float dsc = in ? p * (keep_m * dp - delta_m) * A.sm_scale : 0.f;
+        auto quad = [](float x, auto uc) {
+          return __int_as_float(
+              __builtin_amdgcn_mov_dpp(__float_as_int(x), 0x55 * decltype(uc)::value, 0xf, 0xf, true));
+        };
+        auto add = [&](auto uc) {
+          constexpr int u = decltype(uc)::value;
+          const float cs = quad(dsc, uc), cp = quad(pc, uc);
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) {
+            dk[e] += cs * ElemT<E>::chunk(qd[u], e);
+            dv[e] += cp * ElemT<E>::chunk(gd[u], e);
+          }
+        };
+        add(std::integral_constant<int, 0>{});
+        add(std::integral_constant<int, 1>{});
+        add(std::integral_constant<int, 2>{});
+        add(std::integral_constant<int, 3>{});
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) {
+      dk[e] = slot_sum<LPK>(dk[e]);
+      dv[e] = slot_sum<LPK>(dv[e]);
+    }
+  }
+};
+
+// this lane's 16 bytes of K and V row `key`
+template <Elem E>
+__device__ __forceinline__ void kv_chunks(const GatherBwdArgs& A, int b, int kvh, int key, int ln,
+                                          u32x4& k16, u32x4& v16) {
+  using T = typename ElemT<E>::T;
+  constexpr int EPL = ElemT<E>::kPerChunk;
+  k16 = v16 = u32x4{0u, 0u, 0u, 0u};
+  if (ln * EPL < A.D) {
+    k16 = *(const u32x4*)((const T*)A.k + (int64_t)b * A.ksb + (int64_t)kvh * A.ksh +
+                          (int64_t)key * A.kss + EPL * ln);
+    v16 = *(const u32x4*)((const T*)A.v + (int64_t)b * A.vsb + (int64_t)kvh * A.vsh +
+                          (int64_t)key * A.vss + EPL * ln);
+  }
+}
+
+// A key with more than 2 * part entries is summed in parts, the windows
+// [p part, (p + 1) part) of the sorted order cut to its segment, one wave per
+// window (kv_parts_kernel), and kv_coop_kernel adds the parts in window
+// order: at the last layers every row lists the first keys, and one wave over
+// such a key's q_len entries would outlast the rest of the grid.  A window
+// meets at most two such segments (each longer than two windows): the one
+// holding its first position (slot 2 p) and one starting inside it (2 p + 1).
+template <Elem E, int LPK>
+__global__ __launch_bounds__(256) void kv_parts_kernel(GatherBwdArgs A) {
+  constexpr int EPL = ElemT<E>::kPerChunk;
+  const int lane = threadIdx.x & 63;
+  const int p = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int b = blockIdx.y;
+  if (p >= A.n_windows) return;
+  const int w0 = p * A.part, w1 = (int)min((int64_t)w0 + A.part, A.E);
+  const int sentinel = A.Hkv * A.kv_len;
+  const int g0 = (int)A.keys_out[w0], g1 = (int)A.keys_out[w1 - 1];
+  const int ln = lane % LPK;
+  for (int which = 0; which < 2; ++which) {
+    const int g = which ? g1 : g0;
+    if (g >= sentinel || (which && g1 == g0)) continue;
+    const int i0 = A.seg[g], i1 = A.seg[g + 1];
+    if (i1 - i0 <= 2 * A.part) continue;
+    u32x4 k16, v16;
+    kv_chunks<E>(A, b, g / A.kv_len, g % A.kv_len, ln, k16, v16);
+    KvAcc<E, LPK> acc;
+    acc.clear();
+    acc.run(A, b, k16, v16, max(i0, w0), min(i1, w1), lane);
+    float* dst = A.partial + (((int64_t)b * A.n_windows + p) * 2 + which) * 2 * A.D;
+    if (lane < LPK && ln * EPL < A.D) {
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) {
+        dst[EPL * ln + e] = acc.dk[e];
+        dst[A.D + EPL * ln + e] = acc.dv[e];
+      }
+    }
+  }
+}
+
+template <Elem E, int LPK>
+__global__ __launch_bounds__(256) void kv_coop_kernel(GatherBwdArgs A) {
+  using T = typename ElemT<E>::T;
+  constexpr int EPL = ElemT<E>::kPerChunk;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  // XCD x takes a contiguous range of keys
+  const int blk = (int)(blockIdx.x & 7) * A.keys_per_xcd + (int)(blockIdx.x >> 3);
+  const int64_t gw = (int64_t)blk * 4 + wave;
+  const int b = blockIdx.y;
+  if (gw >= (int64_t)A.Hkv * A.kv_len) return;
+  const int g = (int)gw;
+  const int kvh = g / A.kv_len, key = g % A.kv_len;
+  const int ln = lane % LPK;
+  const int i0 = A.seg[g], i1 = A.seg[g + 1];
+  KvAcc<E, LPK> acc;
+  acc.clear();
+  if (i1 - i0 <= 2 * A.part) {
+    u32x4 k16, v16;
+    kv_chunks<E>(A, b, kvh, key, ln, k16, v16);
+    acc.run(A, b, k16, v16, i0, i1, lane);
+  } else if (ln * EPL < A.D) {
+    for (int p = i0 / A.part; p <= (i1 - 1) / A.part; ++p) {
+      const float* src =
+          A.partial + (((int64_t)b * A.n_windows + p) * 2 + (i0 > p * A.part)) * 2 * A.D;
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) {
+        acc.dk[e] += src[EPL * ln + e];
+        acc.dv[e] += src[A.D + EPL * ln + e];
+      }
+    }
+  }
+  if (lane < LPK && ln * EPL < A.D) {
+    *(u32x4*)((T*)A.dk + (int64_t)b * A.dksb + (int64_t)kvh * A.dksh + (int64_t)key * A.dkss +
+              EPL * ln) = ElemT<E>::pack_chunk(acc.dk);
+    *(u32x4*)((T*)A.dv + (int64_t)b * A.dvsb + (int64_t)kvh * A.dvsh + (int64_t)key * A.dvss +
+              EPL * ln) = ElemT<E>::pack_chunk(acc.dv);
+  }
+}
+
 unsigned grid_for(int64_t n) {
   const int64_t blocks = (n + 255) / 256;
   return (unsigned)(blocks < 65536 ? (blocks > 0 ? blocks : 1) : 65536);
@@ -412,13 +775,99 @@ hipError_t radix_sort(const GatherBwdArgs& A, const uint32_t** keys, const uint3
   return hipSuccess;
 }
 
+// Whether the cooperative-row kernels take the call: 16-byte aligned rows of
+// every tensor, and K / V heads and q / dO batch elements within 32-bit buffer
+// offsets.  Fills what they need in a.
+bool coop_applies(GatherBwdArgs& a, int es) {
+  const int64_t epl = 16 / es;
+  if (a.D % epl != 0) return false;
+  const void* ptrs[] = {a.q, a.k, a.v, a.o, a.dout, a.dq, a.dk, a.dv};
+  for (const void* p : ptrs)
+    if (((uintptr_t)p & 15) != 0) return false;
+  const int64_t st[] = {a.qsb,  a.qsh,  a.qss,  a.ksb,  a.ksh,  a.kss,  a.vsb,  a.vsh,
+                        a.vss,  a.osb,  a.osh,  a.oss,  a.dosb, a.dosh, a.doss, a.dqsb,
+                        a.dqsh, a.dqss, a.dksb, a.dksh, a.dkss, a.dvsb, a.dvsh, a.dvss};
+  for (int64_t x : st)
+    if (x % epl != 0) return false;
+  // bytes from the first to past the last row (n0 rows of stride s0, n1 of
+  // s1); each factor is bounded before it is multiplied
+  auto span = [&](int64_t n0, int64_t s0, int64_t n1, int64_t s1) -> int64_t {
+    if (n0 <= 0 || n1 <= 0) return 0;
+    if (s0 < 0 || s1 < 0 || (n0 > 1 && s0 >= kMaxSpan) || (n1 > 1 && s1 >= kMaxSpan))
+      return kMaxSpan;
+    return ((n0 - 1) * s0 + (n1 - 1) * s1 + a.D) * es;
+  };
+  const int64_t ks = span(a.kv_len, a.kss, 1, 0), vs = span(a.kv_len, a.vss, 1, 0);
+  const int64_t qs = span(a.H, a.qsh, a.q_len, a.qss), gs = span(a.H, a.dosh, a.q_len, a.doss);
+  if (ks >= kMaxSpan || vs >= kMaxSpan || qs >= kMaxSpan || gs >= kMaxSpan) return false;
+  a.k_span = (int)ks;
+  a.v_span = (int)vs;
+  a.q_span = (int)qs;
+  a.do_span = (int)gs;
+  const int64_t rows = (int64_t)a.H * a.q_len;
+  // the per-entry coefficients' 2 B E floats hold the rows' (lse, delta) and
+  // the partial sums of long segments, in windows of at least 512 entries
+  a.ld2 = (float2*)a.cp;
+  const int64_t head = 2 * a.B * rows, left = 2 * a.B * a.E - head;
+  a.partial = a.cp + head;
+  const int64_t per_window = 4 * (int64_t)a.D * a.B;  // floats
+  const int64_t most = left / per_window;             // windows that fit
+  int64_t part = most > 0 ? (a.E + most - 1) / most : a.E;
+  part = (part < 512 ? 512 : part) + 63;
+  part -= part % 64;
+  a.part = (int)(part < (int64_t(1) << 30) ? part : (int64_t(1) << 30));
+  // (segments of more than 2 part entries: none when the grid has no room)
+  a.n_windows = a.E > 2 * (int64_t)a.part ? (int)((a.E + a.part - 1) / a.part) : 0;
+  a.rows_per_xcd = (int)(((rows + 3) / 4 + 7) / 8);
+  a.keys_per_xcd = (int)((((int64_t)a.Hkv * a.kv_len + 3) / 4 + 7) / 8);
+  a.div_w = make_fast_div((uint32_t)a.src.w);
+  a.div_q = make_fast_div((uint32_t)(a.q_len > 0 ? a.q_len : 1));
+  return true;
+}
+
+template <Elem E, int LPK>
+void launch_rows_coop(const GatherBwdArgs& a, bool pattern, hipStream_t stream) {
+  const dim3 grid(8u * (unsigned)a.rows_per_xcd, (unsigned)a.B);
+  if (pattern)
+    rows_coop_kernel<E, LPK, true><<<grid, 256, 0, stream>>>(a);
+  else
+    rows_coop_kernel<E, LPK, false><<<grid, 256, 0, stream>>>(a);
+}
+
+template <Elem E, int LPK>
+void launch_kv_coop(const GatherBwdArgs& a, hipStream_t stream) {
+  if (a.n_windows > 0)
+    kv_parts_kernel<E, LPK>
+        <<<dim3((unsigned)((a.n_windows + 3) / 4), (unsigned)a.B), 256, 0, stream>>>(a);
+  kv_coop_kernel<E, LPK>
+      <<<dim3(8u * (unsigned)a.keys_per_xcd, (unsigned)a.B), 256, 0, stream>>>(a);
+}
+
+// lanes per row: 8, 16, 32 or 64 of 16 bytes (lanes past head_dim idle)
+#define ESA_LANES(E, fn, ...)                             \
+  do {                                                    \
+    const int lanes_ = a.D / ElemT<E>::kPerChunk;         \
+    if (lanes_ <= 8)                                      \
+      fn<E, 8>(__VA_ARGS__);                              \
+    else if (lanes_ <= 16)                                \
+      fn<E, 16>(__VA_ARGS__);                             \
+    else if (lanes_ <= 32)                                \
+      fn<E, 32>(__VA_ARGS__);                             \
+    else if constexpr (ElemT<E>::kPerChunk == 4)          \
+      fn<E, 64>(__VA_ARGS__);                             \
+  } while (0)
+
 template <Elem E>
-hipError_t launch_elem(const GatherBwdArgs& a, bool pattern, hipStream_t stream) {
+hipError_t launch_elem(const GatherBwdArgs& a0, bool pattern, hipStream_t stream) {
+  GatherBwdArgs a = a0;
+  const bool coop = coop_applies(a, ElemT<E>::kBytes);
   GatherBwdArgs s = a;
   hipError_t e = hipSuccess;
   if (a.E > 0) {
     const dim3 rows_grid((unsigned)((a.q_len + 3) / 4), (unsigned)a.H, (unsigned)a.B);
-    if (pattern)
+    if (coop)
+      ESA_LANES(E, launch_rows_coop, a, pattern, stream);
+    else if (pattern)
       bwd_rows_kernel<E, true><<<rows_grid, 256, 0, stream>>>(a);
     else
       bwd_rows_kernel<E, false><<<rows_grid, 256, 0, stream>>>(a);
@@ -441,6 +890,10 @@ hipError_t launch_elem(const GatherBwdArgs& a, bool pattern, hipStream_t stream)
   bwd_segments<<<grid_for((int64_t)a.Hkv * a.kv_len + 1), 256, 0, stream>>>(s);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
+  if (coop) {
+    ESA_LANES(E, launch_kv_coop, s, stream);
+    return hipGetLastError();
+  }
   const dim3 kv_grid((unsigned)((a.kv_len + 3) / 4), (unsigned)a.Hkv, (unsigned)a.B);
   bwd_kv_kernel<E><<<kv_grid, 256, 0, stream>>>(s);
   return hipGetLastError();

@@ -65,7 +65,7 @@ __device__ __forceinline__ float drop_factor(const DropoutArgs& dr, int b, int h
 
 // Sum over aligned groups of N lanes (N = 8, 16, 32, 64), in every lane of
 // the group: DPP within 16-lane rows (quad swaps and a half-row mirror for
-// N = 8, row rotations by 8, 4, 2, 1 for 16), cross-row steps by shuffles.
+// N = 8, row rotations by 8, 4, 2, 1 for 16), cross-row steps by lane swaps.
 template <int N>
 __device__ __forceinline__ float group_sum(float v) {
   auto dpp = [](float x, int ctrl) -> float {
@@ -89,8 +89,16 @@ __device__ __forceinline__ float group_sum(float v) {
   v += dpp(v, 0x124);  // row_ror 4
   v += dpp(v, 0x122);  // row_ror 2
   v += dpp(v, 0x121);  // row_ror 1
-  if (N >= 32) v += __shfl_xor(v, 16, 64);
-  if (N >= 64) v += __shfl_xor(v, 32, 64);
+  if (N >= 32) {
+    const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false,
+                                                    false);
+    v = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+  }
+  if (N >= 64) {
+    const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
+                                                    false);
+    v = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+  }
   return v;
 }
 

@@ -119,6 +119,24 @@ struct GatherArgs {
   int64_t wsb, wsh, wss;
 };
 
+// Division of n < 2^31 by a fixed d >= 1: n / d = (n * mul) >> shift, with
+// mul = floor(2^(31 + s) / d) + 1, s = ceil(log2 d) (Granlund and Montgomery,
+// "Division by invariant integers using multiplication", PLDI 1994):
+// mul * d - 2^(31 + s) is in 1 .. 2^s, so the error n * that / (2^(31 + s) d)
+// stays below 1 / d.
+struct FastDiv {
+  uint32_t mul;
+  int shift;
+};
+inline FastDiv make_fast_div(uint32_t d) {
+  int s = 0;
+  while ((uint64_t(1) << s) < d) ++s;
+  return FastDiv{(uint32_t)((uint64_t(1) << (31 + s)) / d + 1), 31 + s};
+}
+__host__ __device__ inline uint32_t fast_div(uint32_t n, const FastDiv& f) {
+  return (uint32_t)(((uint64_t)n * f.mul) >> f.shift);
+}
+
 // Arguments of the gather backward (any index source, float32 / bfloat16 /
 // float16): per-row pass (dQ and each entry's dK / dV coefficients), a stable
 // sort of the (kv head, key) of every valid entry, then a key-major pass.
@@ -158,6 +176,16 @@ struct GatherBwdArgs {
   int32_t* offs;
   int32_t* parts;     // chunk sums of the scan
   int key_bits;       // bits of the sort keys
+  // the cooperative-row kernels (set by the launcher): (lse, delta) of each
+  // row [B][H q_len] and partial sums [B][n_windows][2][2][D] of long
+  // segments, both in cp / cs's space; bytes spanned by a head's K / V rows and
+  // a batch element's q / dO rows; blocks per XCD range; divisors w and q_len
+  float2* ld2;
+  float* partial;
+  int part, n_windows;
+  int k_span, v_span, q_span, do_span;
+  int rows_per_xcd, keys_per_xcd;
+  FastDiv div_w, div_q;
 };
 
 // Arguments of the block-sparse MFMA backward (bf16).

@@ -161,6 +161,14 @@ def _prep(t: torch.Tensor, align_elems: int) -> torch.Tensor:
     return t
 
 
+def _row_align(t: torch.Tensor) -> int:
+    """The alignment (elements) the gather kernels' 16-byte row loads want of
+    a tensor like ``t``, or 4 (their slower forms) where head_dim rules it
+    out."""
+    n = 16 // t.element_size()
+    return n if t.shape[-1] % n == 0 else 4
+
+
 def make_pattern(seq_len: int, attention_length: int, layer_idx: int, num_hidden_layers: int,
                  num_heads: int, block_m: int = BLOCK_M, block_n: int = BLOCK_N) -> EsaPattern:
     """The pattern parameters the C ABI takes (esa_pattern)."""
@@ -889,8 +897,9 @@ def elastic_attention_bwd_rows(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
     (no atomics on the gradients)."""
     _check_qkv(q, k, v)
     B, H, Lq, D = q.shape
-    q, k, v = _prep(q, 4), _prep(k, 4), _prep(v, 4)
-    dout = _prep(dout.to(q.dtype), 4)
+    align = _row_align(q)
+    q, k, v, o = _prep(q, align), _prep(k, align), _prep(v, align), _prep(o, align)
+    dout = _prep(dout.to(q.dtype), align)
     lse = lse.contiguous()
     dq = torch.empty(B, H, Lq, D, dtype=q.dtype, device=q.device)
     dk = torch.empty_like(k, memory_format=torch.contiguous_format)
@@ -927,8 +936,9 @@ def sparse_attention_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: t
     ``dq``, ``dk``, ``dv`` in the inputs' shapes and dtype; deterministic."""
     _check_qkv(q, k, v)
     B, H, Lq, D = q.shape
-    q, k, v = _prep(q, 4), _prep(k, 4), _prep(v, 4)
-    dout = _prep(dout.to(q.dtype), 4)
+    align = _row_align(q)
+    q, k, v, o = _prep(q, align), _prep(k, align), _prep(v, align), _prep(o, align)
+    dout = _prep(dout.to(q.dtype), align)
     idx, msk = _index_arrays(sparse_indices, sparse_mask)
     dq = torch.empty(B, H, Lq, D, dtype=q.dtype, device=q.device)
     dk = torch.empty_like(k, memory_format=torch.contiguous_format)

@@ -1,0 +1,119 @@
+"""The gather backward's cooperative-row kernels at the sizes where they can
+go wrong: head dims that leave lanes of a row idle, entry counts around the
+chunk of 16 / 32 / 64, keys listed by no row, by one and by more rows than one
+wave sums (the windowed parts), kv groups, dropout; and the slower forms that
+unaligned rows take.
+
+Reference: float64 gradients by autograd through an explicit gather.  Bars:
+float32 1e-5 x max |reference|: a score is a sum of D float32 products, off by
+at most D 2^-24 sum |q k| scale = 0.64 D^1.5 2^-24 (1.6e-4 at D = 256) with every
+rounding aligned, and about 1 / sqrt(D) of that, 1e-5, with independent ones;
+p, and with it the gradients, carry that error as a relative one.  bfloat16 and
+float16: one rounding of the stored gradient, 2^-8 and 2^-11, plus the same
+sums: 6e-3 and 1e-3.
+"""
+import pytest
+import torch
+
+import elastic_sparse_attention as esa
+from elastic_sparse_attention import (elastic_attention_bwd_rows, elastic_attention_rows,
+                                      make_pattern, sparse_attention_bwd, sparse_attention_fwd)
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda", 0)
+BAR = {torch.float32: 1e-5, torch.bfloat16: 6e-3, torch.float16: 1e-3}
+
+
+def inputs(B, H, Hkv, L, D, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    make = lambda h: torch.randn(B, h, L, D, generator=g).to(dtype)  # noqa: E731
+    return make(H), make(Hkv), make(Hkv), make(H), g
+
+
+def reference(q, k, v, go, idx, ok, scale):
+    """float64 dq, dk, dv for explicit lists ``idx`` / ``ok`` [H, L, w]."""
+    q, k, v, go = (t.double().requires_grad_(i < 3) for i, t in enumerate((q, k, v, go)))
+    H, grp = q.shape[1], q.shape[1] // k.shape[1]
+    outs = []
+    for h in range(H):
+        i = torch.where(ok[h], idx[h], torch.zeros_like(idx[h]))
+        kk, vv = k[:, h // grp][:, i], v[:, h // grp][:, i]
+        s = torch.einsum("bld,blwd->blw", q[:, h], kk) * scale
+        p = torch.softmax(s.masked_fill(~ok[h], float("-inf")), -1)
+        outs.append(torch.einsum("blw,blwd->bld", p, vv))
+    o = torch.stack(outs, 1)
+    return torch.autograd.grad(o, (q, k, v), go)
+
+
+def rel(got, ref):
+    return ((got.double().cpu() - ref).abs().max() / ref.abs().max()).item()
+
+
+def check(got, ref, dtype):
+    e = [rel(a, b) for a, b in zip(got, ref)]
+    print("  dq %.2e dk %.2e dv %.2e" % tuple(e), flush=True)
+    assert max(e) <= BAR[dtype]
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 4), (torch.float32, 32), (torch.float32, 60),
+                                     (torch.float32, 128), (torch.float32, 132),
+                                     (torch.float32, 256), (torch.bfloat16, 8),
+                                     (torch.bfloat16, 72), (torch.bfloat16, 128),
+                                     (torch.bfloat16, 256), (torch.bfloat16, 36),
+                                     (torch.float16, 64), (torch.float16, 136)])
+@pytest.mark.parametrize("w", [2, 16, 33, 65])
+def test_operator_head_dims_and_entry_counts(dtype, D, w):
+    B, H, Hkv, L = 2, 4, 2, 67
+    print(f"{dtype} D={D} w={w}", flush=True)
+    q, k, v, go, g = inputs(B, H, Hkv, L, D, dtype, D * 100 + w)
+    idx = torch.randint(0, L, (H, L, w), generator=g)
+    idx[idx == 5] = 6                        # a key no row lists
+    ok = torch.rand(H, L, w, generator=g) > 0.2
+    ok[:, :, 0] = True
+    scale = D ** -0.5
+    d = [t.to(DEV) for t in (q, k, v, idx, ok, go)]
+    o, lse = sparse_attention_fwd(*d[:5], scale, H // Hkv)
+    got = sparse_attention_bwd(*d[:3], o, lse, d[5], d[3], d[4], scale)
+    assert got[1][:, :, 5].abs().max() == 0 and got[2][:, :, 5].abs().max() == 0
+    check(got, reference(q, k, v, go, idx, ok, scale), dtype)
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 64), (torch.bfloat16, 96)])
+@pytest.mark.parametrize("L", [511, 513, 1537])
+def test_keys_that_every_row_lists(dtype, D, L):
+    """Keys 0 and 7 in every row's list (segments of H / Hkv L entries: below,
+    at and above the two windows one wave sums), the rest at random."""
+    B, H, Hkv, w = 2, 4, 2, 12
+    print(f"{dtype} D={D} L={L}", flush=True)
+    q, k, v, go, g = inputs(B, H, Hkv, L, D, dtype, L)
+    idx = torch.randint(0, L, (H, L, w), generator=g)
+    idx[:, :, 3], idx[:, :, 5] = 0, 7
+    ok = torch.ones(H, L, w, dtype=torch.bool)
+    d = [t.to(DEV) for t in (q, k, v, idx, ok, go)]
+    o, lse = sparse_attention_fwd(*d[:5], 0.1, H // Hkv)
+    got = sparse_attention_bwd(*d[:3], o, lse, d[5], d[3], d[4], 0.1)
+    check(got, reference(q, k, v, go, idx, ok, 0.1), dtype)
+    again = sparse_attention_bwd(*d[:3], o, lse, d[5], d[3], d[4], 0.1)
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 64), (torch.bfloat16, 80)])
+@pytest.mark.parametrize("dropout_p", [0.0, 0.3])
+def test_unaligned_rows_agree(dtype, D, dropout_p, monkeypatch):
+    """Rows 4 elements off 16 bytes take the per-lane kernels; both forms
+    give the same gradients to float32 summation order, also with dropout (the
+    same keep decisions)."""
+    B, H, Hkv, L = 2, 4, 2, 700
+    pat = make_pattern(L, 64, 7, 8, H)
+    q, k, v, go, _ = inputs(B, H, Hkv, L, D, dtype, 3)
+    go = go.transpose(1, 2).contiguous()
+    d = [t.to(DEV) for t in (q, k, v)]
+    o, lse = elastic_attention_rows(*d, pat, 0.1, dropout_p=dropout_p, seed=9)
+    want = elastic_attention_bwd_rows(*d, o, lse, go.to(DEV), pat, 0.1, dropout_p=dropout_p,
+                                      seed=9)
+    monkeypatch.setattr(esa, "_row_align", lambda t: 1)  # as given: q one element off
+    off = torch.empty(q.numel() + 1, dtype=dtype, device=DEV)[1:].view(q.shape)
+    off.copy_(d[0])
+    got = elastic_attention_bwd_rows(off, *d[1:], o, lse, go.to(DEV), pat, 0.1,
+                                     dropout_p=dropout_p, seed=9)
+    check(got, [t.double().cpu() for t in want], dtype)
