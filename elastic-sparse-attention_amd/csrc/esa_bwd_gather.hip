@@ -252,39 +252,6 @@ __global__ __launch_bounds__(256) void bwd_kv_kernel(GatherBwdArgs A) {
 // float32 B=2 H=8 L=4096 D=64 467 -> 154 and 564 -> 106 us; bf16 D=96 H=16/4
 // L=5001 496 -> 231 and 1036 -> 236 us.
 
-constexpr uint32_t kOffNone = 0x80000000u;   // an entry's row offset: none
-constexpr uint32_t kLaneNone = 0x7FFFF000u;  // a lane's offset within a row: past head_dim
-// spans stay below both offsets
-constexpr int64_t kMaxSpan = (int64_t(1) << 31) - 8192;
-
-__device__ __forceinline__ u32x4 load16(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
-  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
-}
-
-// v of lane `src` (0 .. 63)
-__device__ __forceinline__ uint32_t from_lane(uint32_t v, int src) {
-  return (uint32_t)__builtin_amdgcn_ds_bpermute(4 * src, (int)v);
-}
-__device__ __forceinline__ float from_lane(float v, int src) {
-  return __uint_as_float(from_lane(__float_as_uint(v), src));
-}
-
-template <Elem E>
-__device__ __forceinline__ float dot16(const u32x4& a, const u32x4& b) {
-  float acc = 0.f;
-#pragma unroll
-  for (int e = 0; e < ElemT<E>::kPerChunk; ++e) acc += ElemT<E>::chunk(a, e) * ElemT<E>::chunk(b, e);
-  return acc;
-}
-
-// sum over the lanes l, l + LPK, l + 2 LPK, ... (a row slot each)
-template <int LPK>
-__device__ __forceinline__ float slot_sum(float v) {
-#pragma unroll
-  for (int off = LPK; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-
 // One wave per (batch, head, query row): dQ and the row's (lse, delta).  A
 // chunk's K and V rows (up to 64 entries) are all in flight before the first
 // score, K stays in registers for dQ, and each lane forms one entry's dS.
@@ -789,13 +756,8 @@ bool coop_applies(GatherBwdArgs& a, int es) {
                         a.dqsh, a.dqss, a.dksb, a.dksh, a.dkss, a.dvsb, a.dvsh, a.dvss};
   for (int64_t x : st)
     if (x % epl != 0) return false;
-  // bytes from the first to past the last row (n0 rows of stride s0, n1 of
-  // s1); each factor is bounded before it is multiplied
-  auto span = [&](int64_t n0, int64_t s0, int64_t n1, int64_t s1) -> int64_t {
-    if (n0 <= 0 || n1 <= 0) return 0;
-    if (s0 < 0 || s1 < 0 || (n0 > 1 && s0 >= kMaxSpan) || (n1 > 1 && s1 >= kMaxSpan))
-      return kMaxSpan;
-    return ((n0 - 1) * s0 + (n1 - 1) * s1 + a.D) * es;
+  auto span = [&](int64_t n0, int64_t s0, int64_t n1, int64_t s1) {
+    return row_span(n0, s0, n1, s1, a.D, es);
   };
   const int64_t ks = span(a.kv_len, a.kss, 1, 0), vs = span(a.kv_len, a.vss, 1, 0);
   const int64_t qs = span(a.H, a.qsh, a.q_len, a.qss), gs = span(a.H, a.dosh, a.q_len, a.doss);

@@ -20,8 +20,8 @@
 // gather_fwd_kernel: lanes split the row's entries 64 at a time for QK (each
 // lane one key, a full dot product over D in float32), then split D for PV
 // (each lane up to four d columns, one 64-key chunk at a time with p and the
-// key broadcast through LDS).  gather_rows_kernel (D = 64, 128, 256 with
-// 16-byte aligned rows) reads each K and V row with D * elem / 16 lanes.
+// key broadcast through LDS).  gather_rows_kernel (16-byte
+// aligned rows) reads each K and V row with a lane per 16 bytes.
 // gather_weights_kernel writes the naive path's attention weights from the
 // forward's lse.
 #include "esa_gather.hpp"
@@ -41,30 +41,35 @@ __global__ __launch_bounds__(256) void gather_fwd_kernel(GatherArgs A) {
 }
 
 // ---------------------------------------------------------------------------
-// Cooperative-row variant for D = 64, 128, 256 with 16-byte aligned rows (the
-// decode shapes): one wave per (batch, head, query row) as above, waves
-// numbered over (batch, head, row) with the row fastest (a one-row decode
-// step fills every wave of a block; a block per row would leave three of
-// its four waves idle), but each
-// K and V row is read by LPK = D * elem / 16 lanes, 16 bytes each, so one
-// load instruction covers KPI = 64 / LPK rows in whole cache lines, and a
-// chunk's K and V rows (SK keys, NI = SK / KPI instructions each) are all in
-// flight before the first score is formed.  Scores: each lane's 16-byte dot
+// Cooperative-row variant for 16-byte aligned rows (head dims of whole 16-byte
+// pieces): one wave per (batch, head, query row) as above, waves numbered over
+// (batch, head, row) with the row fastest (a one-row decode step fills every
+// wave of a block; a block per row would leave three of its four waves idle),
+// but each K and V row is read by LPK lanes (8, 16, 32 or 64: the smallest
+// that hold a row, lanes past head_dim idle), 16 bytes each, so one load
+// instruction covers KPI = 64 / LPK rows in whole cache lines, and a chunk's
+// K and V rows (SK keys, NI = SK / KPI instructions each) are all in flight
+// before the first score is formed.  Scores: each lane's 16-byte dot
 // product, summed over the row's LPK lanes.  PV: each lane accumulates p * V
 // over its 16 bytes of the rows it loaded; the KPI row groups are summed at
 // the end.  Same online softmax, index semantics and float32 accuracy as
 // gather_fwd_kernel (accurate expf; only the order of float32 additions
-// differs).
-template <Elem E, int D, bool PATTERN>
+// differs).  Loads are buffer loads with 32-bit offsets (BUF; a masked entry
+// reads zeros without a fetch) unless a head's K or V spans 2 GiB.
+// XCD x takes a contiguous range of the waves, so its L2 holds the K and V of
+// a few heads: explicit lists bf16 B=2 H=8 L=4096 D=128 200 -> 185 us,
+// float32 D=64 158 -> 151 us, the decode steps unchanged.
+template <Elem E, int LPK, int NMAX, bool BUF, bool PATTERN>
 __global__ __launch_bounds__(256, 2) void gather_rows_kernel(GatherArgs A) {
   __shared__ float sc_all[4][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t wv = (int64_t)blockIdx.x * 4 + wave;
-  // whole wave leaves; no block-level barrier below
-  if (wv >= (int64_t)A.B * A.H * A.q_len) return;
-  const int r = (int)(wv % A.q_len);
-  const int h = (int)((wv / A.q_len) % A.H), b = (int)(wv / ((int64_t)A.q_len * A.H));
-  gather_one_row<E, D, PATTERN>(A, b, h, r, sc_all[wave], lane);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  // XCD x (blockIdx % 8) takes a contiguous range of rows
+  const int wv = (int)(blockIdx.x & 7) * A.waves_per_xcd + (int)(blockIdx.x >> 3) * 4 + wave;
+  if (wv >= A.waves) return;  // whole wave leaves; no block-level barrier below
+  const int bh = wv / A.q_len, r = wv % A.q_len;
+  const int b = bh / A.H, h = bh % A.H;
+  gather_one_row<E, LPK, NMAX, BUF, PATTERN>(A, b, h, r, sc_all[wave], lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -110,11 +115,11 @@ __global__ __launch_bounds__(256) void gather_weights_kernel(GatherArgs A) {
   }
 }
 
-// The cooperative kernel takes D = 64, 128, 256 and needs every Q, K, V and
-// O row 16-byte aligned (bases and strides).
+// The cooperative kernel needs every Q, K, V and O row 16-byte aligned (bases,
+// strides and head_dim).
 bool rows_aligned16(const GatherArgs& a, int es) {
-  if (a.D != 64 && a.D != 128 && a.D != 256) return false;
   const int64_t epl = 16 / es;
+  if (a.D % epl != 0) return false;
   const void* ptrs[] = {a.q, a.k, a.v, a.o};
   for (const void* p : ptrs)
     if (((uintptr_t)p & 15) != 0) return false;
@@ -125,30 +130,52 @@ bool rows_aligned16(const GatherArgs& a, int es) {
   return true;
 }
 
-template <Elem E, bool PATTERN>
-void launch_rows(const GatherArgs& a, dim3 grid, hipStream_t stream) {
-  if (a.D == 64)
-    gather_rows_kernel<E, 64, PATTERN><<<grid, 256, 0, stream>>>(a);
-  else if (a.D == 128)
-    gather_rows_kernel<E, 128, PATTERN><<<grid, 256, 0, stream>>>(a);
+template <Elem E, int LPK, int NMAX, bool BUF>
+void launch_rows(const GatherArgs& a, unsigned blocks, bool pattern, hipStream_t stream) {
+  if (pattern)
+    gather_rows_kernel<E, LPK, NMAX, BUF, true><<<blocks, 256, 0, stream>>>(a);
   else
-    gather_rows_kernel<E, 256, PATTERN><<<grid, 256, 0, stream>>>(a);
+    gather_rows_kernel<E, LPK, NMAX, BUF, false><<<blocks, 256, 0, stream>>>(a);
+}
+
+template <Elem E, int LPK>
+void launch_rows_lanes(const GatherArgs& a, unsigned blocks, bool buf, bool pattern,
+                       hipStream_t stream) {
+  if (buf)
+    launch_rows<E, LPK, 16, true>(a, blocks, pattern, stream);
+  else
+    launch_rows<E, LPK, 16, false>(a, blocks, pattern, stream);
 }
 
 template <Elem E>
 void launch_gather_elem(const GatherArgs& a, bool pattern, hipStream_t stream) {
-  dim3 grid((unsigned)((a.q_len + 3) / 4), (unsigned)a.H, (unsigned)a.B);
   // the cooperative kernel's one-dimensional grid: four waves per block,
   // within the 2^32 work-items of a dispatch
-  const int64_t coop_blocks = ((int64_t)a.B * a.H * a.q_len + 3) / 4;
-  if (rows_aligned16(a, ElemT<E>::kBytes) && coop_blocks * 256 <= (int64_t)UINT32_MAX) {
-    grid = dim3((unsigned)coop_blocks);
-    if (pattern)
-      launch_rows<E, true>(a, grid, stream);
-    else
-      launch_rows<E, false>(a, grid, stream);
+  const int64_t waves = (int64_t)a.B * a.H * a.q_len;
+  const int64_t per_xcd = (waves + 31) / 32;  // blocks
+  if (rows_aligned16(a, ElemT<E>::kBytes) && per_xcd * 8 * 256 <= (int64_t)UINT32_MAX) {
+    GatherArgs c = a;
+    c.waves = (int)waves;  // (< 2^26: the test above)
+    c.waves_per_xcd = (int)per_xcd * 4;
+    const int64_t ks = row_span(a.kv_len, a.kss, 1, 0, a.D, ElemT<E>::kBytes);
+    const int64_t vs = row_span(a.kv_len, a.vss, 1, 0, a.D, ElemT<E>::kBytes);
+    const bool buf = ks < kMaxSpan && vs < kMaxSpan;
+    c.k_span = (int)ks;
+    c.v_span = (int)vs;
+    const unsigned blocks = (unsigned)(8 * per_xcd);
+    // lanes per row: 8, 16, 32 or 64 of 16 bytes (lanes past head_dim idle)
+    const int lanes = a.D / ElemT<E>::kPerChunk;
+    if (lanes <= 8)
+      launch_rows_lanes<E, 8>(c, blocks, buf, pattern, stream);
+    else if (lanes <= 16)
+      launch_rows_lanes<E, 16>(c, blocks, buf, pattern, stream);
+    else if (lanes <= 32)
+      launch_rows_lanes<E, 32>(c, blocks, buf, pattern, stream);
+    else if constexpr (ElemT<E>::kPerChunk == 4)
+      launch_rows_lanes<E, 64>(c, blocks, buf, pattern, stream);
     return;
   }
+  const dim3 grid((unsigned)((a.q_len + 3) / 4), (unsigned)a.H, (unsigned)a.B);
   if (pattern)
     gather_fwd_kernel<E, true><<<grid, 256, 0, stream>>>(a);
   else

@@ -110,43 +110,86 @@ __device__ __forceinline__ void wave_sync_lds() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Row loads through buffer resources, LPK lanes a row: a masked entry, a slot
+// past a list's end or a lane past head_dim gets an offset past num_records
+// and reads zeros without a fetch.
+constexpr uint32_t kOffNone = 0x80000000u;   // an entry's row offset: none
+constexpr uint32_t kLaneNone = 0x7FFFF000u;  // a lane's offset within a row: past head_dim
+// spans stay below both offsets
+constexpr int64_t kMaxSpan = (int64_t(1) << 31) - 8192;
+
+// Bytes from the first to past the last of n0 x n1 rows of D elements (es
+// bytes each) at strides s0, s1, kMaxSpan at least when 32-bit offsets do not
+// reach them (each factor is bounded before it is multiplied)
+inline int64_t row_span(int64_t n0, int64_t s0, int64_t n1, int64_t s1, int D, int es) {
+  if (n0 <= 0 || n1 <= 0) return 0;
+  if (s0 < 0 || s1 < 0 || (n0 > 1 && s0 >= kMaxSpan) || (n1 > 1 && s1 >= kMaxSpan))
+    return kMaxSpan;
+  return ((n0 - 1) * s0 + (n1 - 1) * s1 + D) * es;
+}
+
+__device__ __forceinline__ u32x4 load16(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
+  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
+}
+
+// v of lane `src` (0 .. 63)
+__device__ __forceinline__ uint32_t from_lane(uint32_t v, int src) {
+  return (uint32_t)__builtin_amdgcn_ds_bpermute(4 * src, (int)v);
+}
+__device__ __forceinline__ float from_lane(float v, int src) {
+  return __uint_as_float(from_lane(__float_as_uint(v), src));
+}
+
+// Dot product of two 16-byte chunks
+template <Elem E>
+__device__ __forceinline__ float dot16(const u32x4& a, const u32x4& b) {
+  float acc = 0.f;
+#pragma unroll
+  for (int e = 0; e < ElemT<E>::kPerChunk; ++e) acc += ElemT<E>::chunk(a, e) * ElemT<E>::chunk(b, e);
+  return acc;
+}
+
+// sum over the lanes l, l + LPK, l + 2 LPK, ... (a row slot each)
+template <int LPK>
+__device__ __forceinline__ float slot_sum(float v) {
+#pragma unroll
+  for (int off = LPK; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
 // One query row (b, h, r) of the per-row gather forward, by one wave (the
-// body of gather_rows_kernel, esa_fwd_gather.hip, which describes it; also
-// the band forward's path for rows whose positions are not consecutive):
-// D = 64, 128 or 256 with 16-byte aligned rows; sc: 64 floats of LDS private
-// to the wave.
-template <Elem E, int D, bool PATTERN>
+// body of gather_rows_kernel, esa_fwd_gather.hip, which describes it): LPK
+// lanes read a row of at most LPK 16-byte pieces; NMAX: load instructions of K
+// (and of V) in flight; BUF: K and V by buffer loads (their spans allow it);
+// sc: 64 floats of LDS private to the wave.
+template <Elem E, int LPK, int NMAX, bool BUF, bool PATTERN>
 __device__ __forceinline__ void gather_one_row(const GatherArgs& A, int b, int h, int r,
                                                float* sc, int lane) {
   using T = typename ElemT<E>::T;
   constexpr int EPL = ElemT<E>::kPerChunk;  // elements per lane per load
-  constexpr int LPK = D / EPL;              // lanes per row
   constexpr int KPI = 64 / LPK;             // rows per load instruction
-  constexpr int SK = 16 * KPI < 64 ? 16 * KPI : 64;  // keys per chunk
+  constexpr int SK = NMAX * KPI < 64 ? NMAX * KPI : 64;  // keys per chunk
   constexpr int NI = SK / KPI;              // load instructions per chunk
-  static_assert(LPK <= 64 && 64 % LPK == 0 && NI <= 16, "row split");
+  static_assert(LPK <= 64 && 64 % LPK == 0, "row split");
   const int kvh = h / A.groups;
   const int gk = lane / LPK;  // row of an instruction this lane loads
   const int ln = lane % LPK;  // its 16-byte piece: elements EPL ln .. + EPL
+  const bool act = EPL * ln < A.D;
 
-  float qv[EPL];
-  {
-    const T* qrow = (const T*)A.q + (int64_t)b * A.qsb + (int64_t)h * A.qsh + (int64_t)r * A.qss;
-    const u32x4 raw = *(const u32x4*)(qrow + EPL * ln);
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) qv[e] = ElemT<E>::chunk(raw, e);
-  }
-  const T* kbase = (const T*)A.k + (int64_t)b * A.ksb + (int64_t)kvh * A.ksh + EPL * ln;
-  const T* vbase = (const T*)A.v + (int64_t)b * A.vsb + (int64_t)kvh * A.vsh + EPL * ln;
+  u32x4 q16 = {0u, 0u, 0u, 0u};
+  if (act)
+    q16 = *(const u32x4*)((const T*)A.q + (int64_t)b * A.qsb + (int64_t)h * A.qsh +
+                          (int64_t)r * A.qss + EPL * ln);
+  const T* kbase = (const T*)A.k + (int64_t)b * A.ksb + (int64_t)kvh * A.ksh;
+  const T* vbase = (const T*)A.v + (int64_t)b * A.vsb + (int64_t)kvh * A.vsh;
+  const __amdgpu_buffer_rsrc_t rk =
+      __builtin_amdgcn_make_buffer_rsrc((void*)kbase, (short)0, A.k_span, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rv =
+      __builtin_amdgcn_make_buffer_rsrc((void*)vbase, (short)0, A.v_span, 0x00020000);
+  const uint32_t lofs = act ? 16u * (uint32_t)ln : kLaneNone;
+  const uint32_t kst = (uint32_t)A.kss * sizeof(T), vst = (uint32_t)A.vss * sizeof(T);
   RowEntries row;
   row.init<PATTERN>(A.src, h, r);
-
-  auto dot16 = [&](const u32x4& raw) {
-    float acc = 0.f;
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) acc += qv[e] * ElemT<E>::chunk(raw, e);
-    return acc;
-  };
 
   float m = -INFINITY, l = 0.f;
   float acc[EPL];
@@ -160,17 +203,31 @@ __device__ __forceinline__ void gather_one_row(const GatherArgs& A, int b, int h
     int64_t key = 0;
     if (lane < SK && j < w) row.entry<PATTERN>(A.src, h, r, j, valid, key);
     const bool in_range = key >= 0 && key < A.kv_len;
-    const int kaddr = (valid && in_range) ? (int)key : 0;  // a row that exists
+    const bool live = valid && in_range;
     u32x4 kd[NI], vd[NI];
+    if constexpr (BUF) {
+      const uint32_t ko = live ? (uint32_t)key * kst : kOffNone;
+      const uint32_t vo = live ? (uint32_t)key * vst : kOffNone;
 #pragma unroll
-    for (int t = 0; t < NI; ++t) {
-      const int kk = __shfl(kaddr, KPI * t + gk, 64);
-      kd[t] = *(const u32x4*)(kbase + (int64_t)kk * A.kss);
-      vd[t] = *(const u32x4*)(vbase + (int64_t)kk * A.vss);
+      for (int t = 0; t < NI; ++t) {
+        kd[t] = load16(rk, from_lane(ko, KPI * t + gk) + lofs);
+        vd[t] = load16(rv, from_lane(vo, KPI * t + gk) + lofs);
+      }
+    } else {
+      const uint32_t kaddr = live ? (uint32_t)key : kOffNone;
+#pragma unroll
+      for (int t = 0; t < NI; ++t) {
+        const uint32_t kk = from_lane(kaddr, KPI * t + gk);
+        kd[t] = vd[t] = u32x4{0u, 0u, 0u, 0u};
+        if (act && kk != kOffNone) {
+          kd[t] = *(const u32x4*)(kbase + (int64_t)kk * A.kss + EPL * ln);
+          vd[t] = *(const u32x4*)(vbase + (int64_t)kk * A.vss + EPL * ln);
+        }
+      }
     }
 #pragma unroll
     for (int t = 0; t < NI; ++t) {
-      const float part = group_sum<LPK>(dot16(kd[t]));
+      const float part = group_sum<LPK>(dot16<E>(q16, kd[t]));
       if (ln == 0) sc[KPI * t + gk] = part;
     }
     wave_sync_lds();
@@ -189,7 +246,7 @@ __device__ __forceinline__ void gather_one_row(const GatherArgs& A, int b, int h
     // PV weight of the slot (dropout keep factor applied)
     if (lane < SK) {
       const float keep = j < w ? drop_factor(A.drop, b, h, r, j, A.H, A.q_len, w) : 0.f;
-      sc[lane] = (valid && in_range) ? p * keep : 0.f;
+      sc[lane] = live ? p * keep : 0.f;
     }
     wave_sync_lds();
 #pragma unroll
@@ -202,12 +259,10 @@ __device__ __forceinline__ void gather_one_row(const GatherArgs& A, int b, int h
   }
   // the KPI row groups' partial sums: lanes ln, ln + LPK, ...
 #pragma unroll
-  for (int off = LPK; off < 64; off <<= 1)
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) acc[e] += __shfl_xor(acc[e], off, 64);
+  for (int e = 0; e < EPL; ++e) acc[e] = slot_sum<LPK>(acc[e]);
 
   const float inv = row.bad_pos ? __builtin_nanf("") : (l > 0.f ? 1.f / l : 0.f);
-  if (gk == 0) {
+  if (gk == 0 && act) {
     T* orow = (T*)A.o + (int64_t)b * A.osb + (int64_t)h * A.osh + (int64_t)r * A.oss + EPL * ln;
     float x[EPL];
 #pragma unroll

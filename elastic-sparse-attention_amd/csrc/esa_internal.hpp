@@ -117,6 +117,10 @@ struct GatherArgs {
   // written by launch_gather_weights from the forward's lse)
   void* weights;
   int64_t wsb, wsh, wss;
+  // the cooperative kernel (set by the launcher): bytes a head's K / V rows
+  // span; waves, and waves per XCD range
+  int k_span, v_span;
+  int waves, waves_per_xcd;
 };
 
 // Division of n < 2^31 by a fixed d >= 1: n / d = (n * mul) >> shift, with
