@@ -248,20 +248,20 @@ __global__ __launch_bounds__(256) void bwd_kv_kernel(GatherBwdArgs A) {
 // head_dim gets an offset past num_records and reads zeros without a fetch, so
 // a row that is not listed never meets the sums (no 0 * Inf).  Kernel times,
 // per-lane forms against these: bf16 B=2 H=8 L=4096 D=128 (2.1 GB of rows in
-// each pass) row pass 520 -> 203 us, key pass 787 -> 155 us (13.9 TB/s);
-// float32 B=2 H=8 L=4096 D=64 467 -> 154 and 564 -> 106 us; bf16 D=96 H=16/4
-// L=5001 496 -> 231 and 1036 -> 236 us.
+// each pass) row pass 520 -> 130 us, key pass 787 -> 149 us (14 TB/s);
+// float32 B=2 H=8 L=4096 D=64 467 -> 91 and 564 -> 106 us; bf16 D=96 H=16/4
+// L=5001 496 -> 130 and 1036 -> 226 us.
 
 // One wave per (batch, head, query row): dQ and the row's (lse, delta).  A
-// chunk's K and V rows (up to 64 entries) are all in flight before the first
-// score, K stays in registers for dQ, and each lane forms one entry's dS.
+// chunk's K and V rows are all in flight before the first score, K stays in registers for dQ, and each lane forms one entry's dS.
 // Bound by the L2 row gathers (2 w rows a query row).
 template <Elem E, int LPK, bool PATTERN>
 __global__ __launch_bounds__(256, 2) void rows_coop_kernel(GatherBwdArgs A) {
   using T = typename ElemT<E>::T;
   constexpr int EPL = ElemT<E>::kPerChunk;
   constexpr int KPI = 64 / LPK;
-  constexpr int SK = 16 * KPI < 64 ? 16 * KPI : 64;  // entries per chunk
+  constexpr int NMAX = bwd_in_flight<LPK>();
+  constexpr int SK = NMAX * KPI < 64 ? NMAX * KPI : 64;  // entries per chunk
   constexpr int NI = SK / KPI;
   __shared__ float s_all[4][64];
   __shared__ float dp_all[4][64];

@@ -48,8 +48,8 @@ __global__ __launch_bounds__(256) void gather_fwd_kernel(GatherArgs A) {
 // but each K and V row is read by LPK lanes (8, 16, 32 or 64: the smallest
 // that hold a row, lanes past head_dim idle), 16 bytes each, so one load
 // instruction covers KPI = 64 / LPK rows in whole cache lines, and a chunk's
-// K and V rows (SK keys, NI = SK / KPI instructions each) are all in flight
-// before the first score is formed.  Scores: each lane's 16-byte dot
+// K and V rows (SK keys, NI = SK / KPI <= NMAX instructions each) are all in
+// flight before the first score is formed.  Scores: each lane's 16-byte dot
 // product, summed over the row's LPK lanes.  PV: each lane accumulates p * V
 // over its 16 bytes of the rows it loaded; the KPI row groups are summed at
 // the end.  Same online softmax, index semantics and float32 accuracy as
@@ -138,13 +138,19 @@ void launch_rows(const GatherArgs& a, unsigned blocks, bool pattern, hipStream_t
     gather_rows_kernel<E, LPK, NMAX, BUF, false><<<blocks, 256, 0, stream>>>(a);
 }
 
+// A grid of at most one wave per SIMD (1024) is bound by one wave's latency:
+// there 16 row loads of K and of V are in flight (one row of 32 heads: 7.2
+// against 7.6 us); larger ones take fwd_in_flight (4096 rows 24.5 -> 23.2 us).
 template <Elem E, int LPK>
 void launch_rows_lanes(const GatherArgs& a, unsigned blocks, bool buf, bool pattern,
                        hipStream_t stream) {
-  if (buf)
+  constexpr int NF = fwd_in_flight<E, LPK>();
+  if (!buf)
+    launch_rows<E, LPK, NF, false>(a, blocks, pattern, stream);
+  else if (a.waves <= 1024)
     launch_rows<E, LPK, 16, true>(a, blocks, pattern, stream);
   else
-    launch_rows<E, LPK, 16, false>(a, blocks, pattern, stream);
+    launch_rows<E, LPK, NF, true>(a, blocks, pattern, stream);
 }
 
 template <Elem E>

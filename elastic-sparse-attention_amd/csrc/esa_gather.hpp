@@ -140,12 +140,45 @@ __device__ __forceinline__ float from_lane(float v, int src) {
   return __uint_as_float(from_lane(__float_as_uint(v), src));
 }
 
-// Dot product of two 16-byte chunks
+// Row loads of K (and as many of V) a wave keeps in flight where the grid
+// fills the chip: fewer than a row's list needs, so that more waves share a
+// SIMD (180-210 VGPRs with 16 in flight, 100-140 with 8, 80 with 4) and one
+// wave's sums overlap another's loads.  B=2 H=8 L=4096, 16 / 8 / 4 / 2 in flight,
+// forward (H/Hkv = 4): float32 D=64 148 / 102 / 98 / 132 us, D=128 250 / 170 /
+// 181 / 241, bf16 D=64 73 / 74 / 70 / 83, D=128 158 / 112 / 117 / 138, D=256
+// 296 / 195 / 213 / 267; whole backward: float32 D=64 404 / 356 / 346 / 357,
+// D=256 1116 / 1070 / 1092 / 1154, bf16 D=128 465 / 404 / 395 / 406.
+template <Elem E, int LPK>
+constexpr int fwd_in_flight() {
+  return LPK <= (E == Elem::f32 ? 16 : 8) ? 4 : 8;
+}
+template <int LPK>
+constexpr int bwd_in_flight() {
+  return LPK <= 32 ? 4 : 8;
+}
+
+// Dot product of two 16-byte chunks.  bfloat16 pairs go through v_dot2_f32_bf16
+// (exact products, float32 sums; over 128-element dots of normal values its
+// error against float64 is 7.0e-8, a float32 fma chain's 7.3e-8; Inf, NaN and
+// subnormals as in the chain): 4 instructions instead of 8 conversions and 8
+// fmas (backward row pass bf16 D=128 155 -> 130 us, forward 133 -> 125).
 template <Elem E>
 __device__ __forceinline__ float dot16(const u32x4& a, const u32x4& b) {
   float acc = 0.f;
+  if constexpr (E == Elem::bf16) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-  for (int e = 0; e < ElemT<E>::kPerChunk; ++e) acc += ElemT<E>::chunk(a, e) * ElemT<E>::chunk(b, e);
+    for (int e = 0; e < 4; ++e) {
+      // (copies: a bit cast of a vector's element itself reads element 0)
+      const uint32_t x = a[e], y = b[e];
+      acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, x),
+                                            __builtin_bit_cast(bf16x2, y), acc, false);
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < ElemT<E>::kPerChunk; ++e)
+      acc += ElemT<E>::chunk(a, e) * ElemT<E>::chunk(b, e);
+  }
   return acc;
 }
 
