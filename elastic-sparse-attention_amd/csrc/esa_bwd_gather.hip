@@ -18,11 +18,11 @@
 //                     with a non-finite delta and an entry it does not
 //                     attend gets a NaN dQ, as the Triton kernel's
 //                     (0 - delta) * 0 term for that entry gives it.
-//   bwd_sort_keys     key of each entry: kv_head * kv_len + key for a valid
-//                     in-range entry, else a sentinel past every key.
-//   radix sort        a stable LSD radix sort of (key, entry id), 8 bits per
+//   radix sort        of (key, entry id), the key of an entry being kv_head *
+//                     kv_len + key for a valid in-range entry, else a sentinel
+//                     past every key: a stable LSD radix sort, 8 bits per
 //                     pass (per-tile digit histograms, an exclusive scan of
-//                     them, then a scatter ranked by wave ballots): each
+//                     them, then a scatter ranked by wave ballots), so each
 //                     key's entries end up contiguous, in entry order.
 //   bwd_segments      the start of each (kv head, key) in the sorted order.
 //   bwd_kv_kernel     one wave per (batch, kv head, key): dK = sum of
@@ -137,28 +137,6 @@ __global__ __launch_bounds__(256) void bwd_rows_kernel(GatherBwdArgs A) {
   for (int e = 0; e < 4; ++e) {
     const int d = lane + 64 * e;
     if (d < D) ElemT<E>::store(dqrow + d, all_nan ? __builtin_nanf("") : acc[e]);
-  }
-}
-
-// Sort keys of every entry (batch-independent): kv_head * kv_len + key of a
-// valid entry with a key in [0, kv_len), else the sentinel Hkv * kv_len.
-template <bool PATTERN>
-__global__ __launch_bounds__(256) void bwd_sort_keys(GatherBwdArgs A) {
-  const int w = A.src.w;
-  const uint32_t sentinel = (uint32_t)A.Hkv * (uint32_t)A.kv_len;
-  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < A.E;
-       e += (int64_t)gridDim.x * 256) {
-    const int j = (int)(e % w);
-    const int64_t hr = e / w;
-    const int r = (int)(hr % A.q_len), h = (int)(hr / A.q_len);
-    RowEntries row;
-    row.init<PATTERN>(A.src, h, r);
-    bool valid = false;
-    int64_t key = 0;
-    row.entry<PATTERN>(A.src, h, r, j, valid, key);
-    const bool live = valid && key >= 0 && key < A.kv_len && !row.bad_pos;
-    A.keys_in[e] = live ? (uint32_t)(h / A.groups) * (uint32_t)A.kv_len + (uint32_t)key : sentinel;
-    A.vals_in[e] = (uint32_t)e;
   }
 }
 
@@ -567,12 +545,46 @@ unsigned grid_for(int64_t n) {
 }
 
 // ---------------------------------------------------------------------------
-// Stable LSD radix sort of (uint32 key, uint32 value) pairs, 8 bits a pass.
+// Stable LSD radix sort of (uint32 key, uint32 entry id) pairs, 8 bits a pass.
 // A tile is 4096 pairs: wave w of a 256-thread block owns tile positions
 // [1024 w, 1024 (w + 1)), item i and lane l holding position 1024 w + 64 i + l,
-// so (wave, item, lane) order is the input order.
+// so (wave, item, lane) order is the input order.  Three launches a pass:
+// digit counts per tile (the first pass forms the keys there), their scan (a
+// block per digit) and the scatter.  2.1M pairs with 16-bit keys, the launches
+// of both passes: 125 -> 60 us against one-pair-at-a-time stores and separate
+// key and chunked-scan launches (first scatter 52 -> 16 us); 5.1M: 230 -> 105.
 constexpr int kSortTile = 4096;
-constexpr int kScanChunk = 2048;
+constexpr int kScanChunk = 2048;  // of the workspace's size formula
+
+// Sort keys of every entry (batch-independent): kv_head * kv_len + key of a
+// valid entry with a key in [0, kv_len), else the sentinel Hkv * kv_len; and
+// hist[d * nb + blk] = entries of tile blk whose lowest digit is d
+template <bool PATTERN>
+__global__ __launch_bounds__(256) void sort_keys_hist(GatherBwdArgs A, int nb) {
+  __shared__ int cnt[256];
+  cnt[threadIdx.x] = 0;
+  __syncthreads();
+  const uint32_t sentinel = (uint32_t)A.Hkv * (uint32_t)A.kv_len;
+  const int64_t t0 = (int64_t)blockIdx.x * kSortTile;
+  for (int i = threadIdx.x; i < kSortTile && t0 + i < A.E; i += 256) {
+    const uint32_t e = (uint32_t)(t0 + i);
+    const uint32_t hr = fast_div(e, A.div_w);
+    const int j = (int)(e - hr * (uint32_t)A.src.w);
+    const int h = (int)fast_div(hr, A.div_q), r = (int)(hr - (uint32_t)h * (uint32_t)A.q_len);
+    RowEntries row;
+    row.init<PATTERN>(A.src, h, r);
+    bool valid = false;
+    int64_t key = 0;
+    row.entry<PATTERN>(A.src, h, r, j, valid, key);
+    const bool live = valid && key >= 0 && key < A.kv_len && !row.bad_pos;
+    const uint32_t k =
+        live ? (uint32_t)(h / A.groups) * (uint32_t)A.kv_len + (uint32_t)key : sentinel;
+    A.keys_in[e] = k;
+    atomicAdd(&cnt[k & 255u], 1);
+  }
+  __syncthreads();
+  A.hist[(int64_t)threadIdx.x * nb + blockIdx.x] = cnt[threadIdx.x];
+}
 
 // hist[d * nb + blk] = pairs of tile blk whose digit is d
 __global__ __launch_bounds__(256) void radix_hist(const uint32_t* __restrict__ keys, int64_t n,
@@ -608,75 +620,49 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* buf, int* total)
   return incl - v;
 }
 
-// parts[c] = sum of chunk c of x (kScanChunk entries)
-__global__ __launch_bounds__(256) void scan_chunk_sums(const int32_t* __restrict__ x, int64_t n,
-                                                       int32_t* __restrict__ parts) {
+// offs[d * nb + blk] = pairs of digit d in tiles before blk (one block a digit)
+__global__ __launch_bounds__(256) void radix_scan(const int32_t* __restrict__ hist, int nb,
+                                                  int32_t* __restrict__ offs) {
   __shared__ int buf[256];
-  const int64_t c0 = (int64_t)blockIdx.x * kScanChunk;
-  int v = 0;
-  for (int i = threadIdx.x; i < kScanChunk; i += 256)
-    if (c0 + i < n) v += x[c0 + i];
-  int total = 0;
-  block_exclusive_scan(v, buf, &total);
-  if (threadIdx.x == 0) parts[blockIdx.x] = total;
-}
-
-// exclusive scan of the chunk sums in place (one block)
-__global__ __launch_bounds__(256) void scan_parts(int32_t* __restrict__ parts, int np) {
-  __shared__ int buf[256];
+  const int64_t row = (int64_t)blockIdx.x * nb;
   int carry = 0;
-  for (int base = 0; base < np; base += 256) {
+  for (int base = 0; base < nb; base += 256) {
     const int i = base + threadIdx.x;
-    const int v = i < np ? parts[i] : 0;
+    const int v = i < nb ? hist[row + i] : 0;
     int total = 0;
     const int ex = block_exclusive_scan(v, buf, &total);
-    if (i < np) parts[i] = carry + ex;
+    if (i < nb) offs[row + i] = carry + ex;
     carry += total;
   }
 }
 
-// out = exclusive scan of x: each chunk scanned in the block (eight
-// consecutive entries per thread), plus its chunk's prefix
-__global__ __launch_bounds__(256) void scan_apply(const int32_t* __restrict__ x, int64_t n,
-                                                  const int32_t* __restrict__ parts,
-                                                  int32_t* __restrict__ out) {
-  __shared__ int buf[256];
-  constexpr int PER = kScanChunk / 256;
-  const int64_t c0 = (int64_t)blockIdx.x * kScanChunk + (int64_t)threadIdx.x * PER;
-  int v[PER];
-  int sum = 0;
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    v[k] = c0 + k < n ? x[c0 + k] : 0;
-    sum += v[k];
-  }
-  int total = 0;
-  int run = block_exclusive_scan(sum, buf, &total) + parts[blockIdx.x];
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    if (c0 + k < n) out[c0 + k] = run;
-    run += v[k];
-  }
-}
-
-// Scatter of one pass: a pair goes to offs[d * nb + blk] + (pairs of digit d
-// in earlier waves of the tile) + (pairs of digit d before it in its wave).
-// Ranks within a wave come from eight ballots per item (the lanes sharing
-// the pair's digit) and per-wave running digit counts in LDS.
+// Scatter of one pass: a pair goes to (pairs of smaller digits) + offs[d * nb
+// + blk] + (pairs of digit d in earlier waves of the tile) + (pairs of digit d
+// before it in its wave).  Ranks within a wave come from eight ballots per
+// item (the lanes sharing the pair's digit) and per-wave running digit counts
+// in LDS.  The tile is put in order in LDS first, so the stores go out in runs
+// of equal digits instead of one pair at a time.  FIRST: entry ids are the
+// input positions.
+template <bool FIRST>
 __global__ __launch_bounds__(256) void radix_scatter(const uint32_t* __restrict__ kin,
                                                      const uint32_t* __restrict__ vin, int64_t n,
                                                      int shift, int nb,
+                                                     const int32_t* __restrict__ hist,
                                                      const int32_t* __restrict__ offs,
                                                      uint32_t* __restrict__ kout,
                                                      uint32_t* __restrict__ vout) {
   __shared__ int cnt[4][256];
+  __shared__ int buf[256];
+  __shared__ int base_g[256];  // global position of the digit's first pair, minus its local one
+  __shared__ uint32_t lk[kSortTile], lv[kSortTile];
   constexpr int ITEMS = kSortTile / 256;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int blk = blockIdx.x;
   for (int i = threadIdx.x; i < 4 * 256; i += 256) (&cnt[0][0])[i] = 0;
   __syncthreads();
   const uint64_t below = lane ? (~0ull >> (64 - lane)) : 0ull;
-  const int64_t p0 = (int64_t)blk * kSortTile + (int64_t)wave * (64 * ITEMS);
+  const int64_t t0 = (int64_t)blk * kSortTile;
+  const int64_t p0 = t0 + (int64_t)wave * (64 * ITEMS);
   uint32_t key[ITEMS], val[ITEMS];
   int rank[ITEMS];
 #pragma unroll
@@ -684,7 +670,11 @@ __global__ __launch_bounds__(256) void radix_scatter(const uint32_t* __restrict_
     const int64_t x = p0 + (int64_t)it * 64 + lane;
     const bool ok = x < n;
     key[it] = ok ? kin[x] : 0u;
-    val[it] = ok ? vin[x] : 0u;
+    val[it] = FIRST ? (uint32_t)x : ok ? vin[x] : 0u;
+  }
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    const bool ok = p0 + (int64_t)it * 64 + lane < n;
     const uint32_t d = (key[it] >> shift) & 255u;
     uint64_t peers = __builtin_amdgcn_ballot_w64(ok);
 #pragma unroll
@@ -700,38 +690,66 @@ __global__ __launch_bounds__(256) void radix_scatter(const uint32_t* __restrict_
     wave_sync_lds();
   }
   __syncthreads();
+  // thread d: its digit's pairs in the tile and in the whole input, both
+  // scanned over the digits; cnt[w][d] becomes the local position of the
+  // digit's first pair of wave w
+  {
+    const int d = threadIdx.x;
+    int c[4];
+#pragma unroll
+    for (int w2 = 0; w2 < 4; ++w2) c[w2] = cnt[w2][d];
+    const int64_t row = (int64_t)d * nb;
+    const int all = offs[row + nb - 1] + hist[row + nb - 1];
+    int total = 0;
+    int at = block_exclusive_scan(c[0] + c[1] + c[2] + c[3], buf, &total);
+    const int first = block_exclusive_scan(all, buf, &total);
+    base_g[d] = first + offs[row + blk] - at;
+#pragma unroll
+    for (int w2 = 0; w2 < 4; ++w2) {
+      cnt[w2][d] = at;
+      at += c[w2];
+    }
+  }
+  __syncthreads();
 #pragma unroll
   for (int it = 0; it < ITEMS; ++it) {
-    const int64_t x = p0 + (int64_t)it * 64 + lane;
-    if (x >= n) continue;
-    const uint32_t d = (key[it] >> shift) & 255u;
-    int before = 0;
-    for (int w2 = 0; w2 < wave; ++w2) before += cnt[w2][d];
-    const int64_t dst = (int64_t)offs[(int64_t)d * nb + blk] + before + rank[it];
-    kout[dst] = key[it];
-    vout[dst] = val[it];
+    if (p0 + (int64_t)it * 64 + lane >= n) continue;
+    const int at = cnt[wave][(key[it] >> shift) & 255u] + rank[it];
+    lk[at] = key[it];
+    lv[at] = val[it];
+  }
+  __syncthreads();
+  const int here = (int)(n - t0 < kSortTile ? n - t0 : kSortTile);
+  for (int i = threadIdx.x; i < here; i += 256) {
+    const uint32_t k = lk[i];
+    const int dst = base_g[(k >> shift) & 255u] + i;
+    kout[dst] = k;
+    vout[dst] = lv[i];
   }
 }
 
-// Sorts (A.keys_in, A.vals_in) over the low key_bits bits; returns, through
-// *keys / *vals, the buffers holding the result (the pair buffers alternate
-// by pass).
-hipError_t radix_sort(const GatherBwdArgs& A, const uint32_t** keys, const uint32_t** vals,
-                      hipStream_t stream) {
+// Sorts the entries by key over the low key_bits bits; returns, through *keys
+// / *vals, the buffers holding the result (the pair buffers alternate by pass).
+hipError_t radix_sort(const GatherBwdArgs& A, bool pattern, const uint32_t** keys,
+                      const uint32_t** vals, hipStream_t stream) {
   const int64_t n = A.E;
   const int nb = (int)((n + kSortTile - 1) / kSortTile);
-  const int64_t nh = (int64_t)256 * nb;
-  const int np = (int)((nh + kScanChunk - 1) / kScanChunk);
   uint32_t* ka = A.keys_in;
   uint32_t* va = A.vals_in;
   uint32_t* kb = A.keys_out;
   uint32_t* vb = A.vals_out;
   for (int shift = 0; shift < A.key_bits; shift += 8) {
-    radix_hist<<<nb, 256, 0, stream>>>(ka, n, shift, nb, A.hist);
-    scan_chunk_sums<<<np, 256, 0, stream>>>(A.hist, nh, A.parts);
-    scan_parts<<<1, 256, 0, stream>>>(A.parts, np);
-    scan_apply<<<np, 256, 0, stream>>>(A.hist, nh, A.parts, A.offs);
-    radix_scatter<<<nb, 256, 0, stream>>>(ka, va, n, shift, nb, A.offs, kb, vb);
+    if (shift > 0)
+      radix_hist<<<nb, 256, 0, stream>>>(ka, n, shift, nb, A.hist);
+    else if (pattern)
+      sort_keys_hist<true><<<nb, 256, 0, stream>>>(A, nb);
+    else
+      sort_keys_hist<false><<<nb, 256, 0, stream>>>(A, nb);
+    radix_scan<<<256, 256, 0, stream>>>(A.hist, nb, A.offs);
+    if (shift > 0)
+      radix_scatter<false><<<nb, 256, 0, stream>>>(ka, va, n, shift, nb, A.hist, A.offs, kb, vb);
+    else
+      radix_scatter<true><<<nb, 256, 0, stream>>>(ka, va, n, shift, nb, A.hist, A.offs, kb, vb);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     uint32_t* t = ka; ka = kb; kb = t;
@@ -782,8 +800,6 @@ bool coop_applies(GatherBwdArgs& a, int es) {
   a.n_windows = a.E > 2 * (int64_t)a.part ? (int)((a.E + a.part - 1) / a.part) : 0;
   a.rows_per_xcd = (int)(((rows + 3) / 4 + 7) / 8);
   a.keys_per_xcd = (int)((((int64_t)a.Hkv * a.kv_len + 3) / 4 + 7) / 8);
-  a.div_w = make_fast_div((uint32_t)a.src.w);
-  a.div_q = make_fast_div((uint32_t)(a.q_len > 0 ? a.q_len : 1));
   return true;
 }
 
@@ -822,6 +838,8 @@ void launch_kv_coop(const GatherBwdArgs& a, hipStream_t stream) {
 template <Elem E>
 hipError_t launch_elem(const GatherBwdArgs& a0, bool pattern, hipStream_t stream) {
   GatherBwdArgs a = a0;
+  a.div_w = make_fast_div((uint32_t)a.src.w);
+  a.div_q = make_fast_div((uint32_t)(a.q_len > 0 ? a.q_len : 1));
   const bool coop = coop_applies(a, ElemT<E>::kBytes);
   GatherBwdArgs s = a;
   hipError_t e = hipSuccess;
@@ -835,15 +853,9 @@ hipError_t launch_elem(const GatherBwdArgs& a0, bool pattern, hipStream_t stream
       bwd_rows_kernel<E, false><<<rows_grid, 256, 0, stream>>>(a);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if (pattern)
-      bwd_sort_keys<true><<<grid_for(a.E), 256, 0, stream>>>(a);
-    else
-      bwd_sort_keys<false><<<grid_for(a.E), 256, 0, stream>>>(a);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
     const uint32_t* sk = nullptr;
     const uint32_t* sv = nullptr;
-    e = radix_sort(a, &sk, &sv, stream);
+    e = radix_sort(a, pattern, &sk, &sv, stream);
     if (e != hipSuccess) return e;
     s.keys_out = const_cast<uint32_t*>(sk);
     s.vals_out = const_cast<uint32_t*>(sv);

@@ -175,10 +175,10 @@ esa_status hip_status(hipError_t e) { return e == hipSuccess ? ESA_OK : ESA_ERR_
 // Byte offsets of the gather backward's workspace regions (each 256-byte
 // aligned): per batch element and entry a dV and a dK coefficient, two
 // (key, entry id) pair buffers for the sort, the per-key segment starts and
-// the sort's digit histograms, their scan and its chunk sums.
+// the sort's digit histograms and their scan.
 struct GatherBwdLayout {
   int64_t E;  // entries per batch element: H * q_len * w
-  size_t cp, cs, ka, va, kb, vb, seg, hist, offs, parts, total;
+  size_t cp, cs, ka, va, kb, vb, seg, hist, offs, total;
 };
 
 esa_status gather_bwd_layout(const esa_bwd_args* a, int32_t w, GatherBwdLayout* L) {
@@ -208,7 +208,7 @@ esa_status gather_bwd_layout(const esa_bwd_args* a, int32_t w, GatherBwdLayout* 
   L->seg = take(((size_t)a->num_kv_heads * a->kv_len + 1) * 4);
   L->hist = take((size_t)hist_ints * 4);
   L->offs = take((size_t)hist_ints * 4);
-  L->parts = take((size_t)part_ints * 4);
+  take((size_t)part_ints * 4);  // spare: the size that callers allocate stays the same
   L->total = at;
   return ESA_OK;
 }
@@ -274,7 +274,6 @@ esa_status gather_bwd_args(const esa_bwd_args* a, int32_t w, void* workspace,
   t.seg = (int32_t*)(ws + L.seg);
   t.hist = (int32_t*)(ws + L.hist);
   t.offs = (int32_t*)(ws + L.offs);
-  t.parts = (int32_t*)(ws + L.parts);
   int bits = 1;
   while (bits < 32 && ((uint64_t)1 << bits) <= (uint64_t)a->num_kv_heads * a->kv_len) ++bits;
   t.key_bits = bits;  // the sentinel Hkv * kv_len fits

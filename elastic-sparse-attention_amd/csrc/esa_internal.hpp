@@ -172,13 +172,12 @@ struct GatherBwdArgs {
   float* cp;          // [B][E] dV coefficient of each entry (dropout-scaled p)
   float* cs;          // [B][E] dK coefficient of each entry (sm_scale * dS)
   uint32_t* keys_in;  // [E] kv_head * kv_len + key of a valid in-range entry, else the sentinel
-  uint32_t* vals_in;  // [E] entry ids 0 .. E - 1
+  uint32_t* vals_in;  // [E] entry ids
   uint32_t* keys_out;
   uint32_t* vals_out;
   int32_t* seg;       // [Hkv * kv_len + 1] start of each (kv head, key) in the sorted order
   int32_t* hist;      // radix sort: digit counts per tile, then their scan (offs)
   int32_t* offs;
-  int32_t* parts;     // chunk sums of the scan
   int key_bits;       // bits of the sort keys
   // the cooperative-row kernels (set by the launcher): (lse, delta) of each
   // row [B][H q_len] and partial sums [B][n_windows][2][2][D] of long
@@ -189,7 +188,7 @@ struct GatherBwdArgs {
   int part, n_windows;
   int k_span, v_span, q_span, do_span;
   int rows_per_xcd, keys_per_xcd;
-  FastDiv div_w, div_q;
+  FastDiv div_w, div_q;  // (set for every call)
 };
 
 // Arguments of the block-sparse MFMA backward (bf16).
@@ -293,8 +292,8 @@ hipError_t launch_band_dkdv(const BwdArgs& a, int head_dim, const float* lse2,
                             hipStream_t stream);
 hipError_t launch_gather_fwd(const GatherArgs& a, bool pattern, hipStream_t stream);
 hipError_t launch_gather_weights(const GatherArgs& a, bool pattern, hipStream_t stream);
-// int32 entries of the sort's digit histograms (and of their scan) and of
-// its scan's chunk sums, for n pairs
+// int32 entries of the sort's digit histograms (and of their scan), and a
+// spare region's (one per 2048 of them), for n pairs
 void gather_bwd_sort_sizes(int64_t n, int64_t* hist_ints, int64_t* part_ints);
 hipError_t launch_gather_bwd(const GatherBwdArgs& a, bool pattern, hipStream_t stream);
 hipError_t launch_tile_masks(const PatternConsts& pc, const int32_t* row_ptr, const int32_t* col_idx,
