@@ -16,6 +16,31 @@ namespace esa {
 
 typedef __attribute__((address_space(3))) uint16_t lds_u16;
 
+// The (batch, head, row group) of group g.  inner = 1: a query head's row
+// groups one after another, heads outermost; inner = groups: the query heads
+// that share a K and V run fastest, row groups next, so the groups an XCD
+// holds at once read the keys of fewer rows (the callers say where that pays).
+struct GroupId {
+  int b, h, kvh, gq;
+};
+__device__ __forceinline__ GroupId group_id(int g, int ng, int inner, int H, int groups) {
+  GroupId r;
+  if (inner == 1) {
+    const int bh = g / ng;
+    r.gq = g % ng;
+    r.h = bh % H;
+    r.b = bh / H;
+  } else {
+    const int per = ng * inner, outer = H / inner;
+    const int bo = g / per, rem = g % per;
+    r.gq = rem / inner;
+    r.b = bo / outer;
+    r.h = bo % outer * inner + rem % inner;
+  }
+  r.kvh = r.h / groups;
+  return r;
+}
+
 template <int D>
 struct BandCfg {
   static constexpr int NS = D / 32;       // QK^T k-steps (32 dims each)

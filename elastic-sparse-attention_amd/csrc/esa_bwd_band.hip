@@ -53,9 +53,8 @@ __global__ __launch_bounds__(64, 2) void band_dq_kernel(BwdArgs A, const float* 
   const int bid = blockIdx.x;
   const int g = (bid & 7) * A.per_xcd + (bid >> 3);
   if (g >= A.n_groups) return;
-  const int bh = g / A.ng, gq = g % A.ng;
-  const int h = bh % A.H, b = bh / A.H;
-  const int kvh = h / A.groups;
+  const GroupId id = group_id(g, A.ng, 1, A.H, A.groups);
+  const int b = id.b, h = id.h, kvh = id.kvh, gq = id.gq;
 
   const int lane = threadIdx.x;
   const int n = lane & 15, q = lane >> 4;
@@ -401,7 +400,7 @@ __global__ __launch_bounds__(64, 2) void band_dq_kernel(BwdArgs A, const float* 
   // group exactly)
   {
     const bool bad = wave_any(!sum_finite(dqacc));
-    if (lane == 0) A.flags[g] = bad ? 1 : 0;
+    if (lane == 0) A.flags[((int64_t)b * A.H + h) * A.ng + gq] = bad ? 1 : 0;
   }
   // ---- dQ = scale * dQ^T^T: lane (n, q) holds dims CW q + 4 s + e of row n
   if (row_ok) {
@@ -458,9 +457,8 @@ __global__ __launch_bounds__(64, 2) void window_dq_kernel(BwdArgs A, const float
   const int bid = blockIdx.x;
   const int g = (bid & 7) * per2 + (bid >> 3);
   if (g >= n2) return;
-  const int bh = g / ng2, gq = g % ng2;
-  const int h = bh % A.H, b = bh / A.H;
-  const int kvh = h / A.groups;
+  const GroupId id = group_id(g, ng2, A.win_inner, A.H, A.groups);
+  const int b = id.b, h = id.h, kvh = id.kvh, gq = id.gq;
 
   const int lane = threadIdx.x;
   const int n = lane & 15, q = lane >> 4;
@@ -698,7 +696,7 @@ __global__ __launch_bounds__(64, 2) void window_dq_kernel(BwdArgs A, const float
     // the 16-row group's non-finite flag (see band_dq_kernel)
     const int g16 = 2 * gq + u;
     const bool bad = wave_any(!sum_finite(dqacc[u]));
-    if (lane == 0 && g16 < A.ng) A.flags[(int64_t)bh * A.ng + g16] = bad ? 1 : 0;
+    if (lane == 0 && g16 < A.ng) A.flags[((int64_t)b * A.H + h) * A.ng + g16] = bad ? 1 : 0;
     const int i = r0 + 16 * u + n;
     if (i < A.q_len) {
       uint16_t* dqr = A.dq + (int64_t)b * A.dqsb + (int64_t)h * A.dqsh + (int64_t)i * A.dqss;
@@ -1225,7 +1223,12 @@ static void launch_band_dq_d(const BwdArgs& a, dim3 grid, const float* lse2, hip
   if (a.pc.a == 0.0f) {
     // 32-row groups (window_dq_kernel), XCD-contiguous like the 16-row grid
     const int64_t n2 = (int64_t)a.B * a.H * ((a.q_len + 31) / 32);
-    window_dq_kernel<D, PREP, E><<<dim3((unsigned)(8 * ((n2 + 7) / 8))), 64, 0, stream>>>(a, lse2);
+    // the heads of a kv group together where a head's K and V fill an XCD's
+    // L2 (group_id): B=1 H=32/8 L=32768 D=128 backward 642 -> 608 us, H=32/4
+    // L=8192 150 -> 146; below that 0-2% slower (B=8 H=16/4 L=4096 D=64 153 -> 157)
+    BwdArgs w = a;
+    w.win_inner = (int64_t)a.kv_len * 4 * D >= (int64_t(4) << 20) ? a.groups : 1;
+    window_dq_kernel<D, PREP, E><<<dim3((unsigned)(8 * ((n2 + 7) / 8))), 64, 0, stream>>>(w, lse2);
   } else if (a.pc.a >= 0.5f)
     band_dq_kernel<D, true, PREP, E><<<grid, 64, 0, stream>>>(a, lse2);
   else

@@ -94,9 +94,8 @@ __global__ __launch_bounds__(64 * S, 2) void band_fwd_kernel(BandArgs A) {
   const int bid = blockIdx.x;
   const int g = (bid & 7) * A.per_xcd + (bid >> 3);
   if (g >= A.n_groups) return;
-  const int bh = g / A.ng, gq = g % A.ng;
-  const int h = bh % A.H, b = bh / A.H;
-  const int kvh = h / A.groups;
+  const GroupId id = group_id(g, A.ng, A.inner, A.H, A.groups);
+  const int b = id.b, h = id.h, kvh = id.kvh, gq = id.gq;
 
   const int lane = S > 1 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
   const int n = lane & 15, q = lane >> 4;
@@ -747,9 +746,23 @@ hipError_t launch_band_fwd(const BandArgs& a, int head_dim, hipStream_t stream) 
   // layers 4 and 7, the late 32768-row chunks of L=131072 6-34%, early
   // chunks (position 0) within 1%; full prefills at 6.4 rounds up to 15%
   // slower, and late chunks at layer 2 of L=131072 18-36% slower.
-  const int max_rounds = a.positions && a.pc.a >= 0.5f ? 8 : 4;
+  // With four or more query heads to a kv head these few-round chunks also run
+  // such heads together (inner, below), which divides the keys a round works
+  // on, and both limits double.
+  const int max_rounds = (a.positions && a.pc.a >= 0.5f ? 8 : 4) *
+                         (a.positions && a.groups >= 4 ? 2 : 1);
   r.rot_rate = band_rotation(a.n_groups, 40960 / dk, (int64_t)a.kv_len * 4 * a.d_real,
                              dk == 128 ? 15 : 9, 3, max_rounds);
+  // The query heads of a kv group together (group_id) in the chunks that
+  // rotate by `few`: their rows' keys exceed L2 one head after another.  Late
+  // chunks, heads in turn against together: H=32/4 L=65536 D=128 4096 rows
+  // layer 3 / 4 / 7 237 / 264 / 189 -> 168 / 160 / 176 us, 8192 rows 460 / 631
+  // / 470 -> 320 / 309 / 335, 16384 rows layers 4 / 7 (the doubled limit) 898 /
+  // 1003 -> 616 / 654; H=32/8 L=100000 8192 rows 753 -> 354; H=32/16 L=65536
+  // 8192 rows 633 -> 511; early chunks and D=64 within 2%.  At layer 2 of
+  // L=100000 16384 rows were 7% slower with a limit of 16 rounds, and H=32/16
+  // there 11-15%.  Full prefills of few heads: between -7% (layer 1) and +2%.
+  r.inner = a.positions && r.rot_rate == 3 ? a.groups : 1;
   // K DMA skipping: with the late V order from interpolation weight 1/2 on
   // (measured at B=1, H=32, L=32768, D=128, w=64 over 8 layers: 1-7% faster
   // at weights 4/7 .. 1, even at 3/7, 3-4% slower at 1/7 and 2/7, where

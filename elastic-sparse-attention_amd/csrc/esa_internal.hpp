@@ -68,8 +68,9 @@ struct BandArgs {
   // dims d_real .. D - 1 of Q, K and V read as zeros and O's are not stored
   int d_real;
   // entry rotation of the band forward, in 64ths of an entry per group
-  // dispatched on an XCD (set by launch_band_fwd from the grid's size)
-  int rot_rate;
+  // dispatched on an XCD, and the query heads run together (group_id; both set
+  // by launch_band_fwd from the grid's size)
+  int rot_rate, inner;
 };
 
 // Where a query row's w entries come from: the elastic pattern (regenerated
@@ -250,6 +251,8 @@ struct BwdArgs {
   // entry rotation of the band dQ / dK-dV walks, in 64ths of an entry per
   // group or block dispatched on an XCD (set by their launchers)
   int rot_dq, rot_dkdv;
+  // query heads the window dQ runs together (group_id; set by its launcher)
+  int win_inner;
 };
 
 // Entry rotation rate of a band kernel's launch (64ths of an entry per unit
