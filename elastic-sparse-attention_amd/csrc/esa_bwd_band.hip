@@ -757,23 +757,32 @@ __global__ __launch_bounds__(64, 2) void window_dq_kernel(BwdArgs A, const float
 // order and writes the block, so results do not depend on which wave is
 // last.
 //
+// S: waves per block (band_dkdv_waves): the group's query heads, or every
+// head's steps where the heads do not divide, are shared out, each wave
+// accumulates in registers through slots of its own, and wave 0 adds the sums
+// in wave order.
+//
 // WIN: interpolation weight 0 (layer 0, a sliding window).  Key u is
 // attended by rows u .. u + w - 1, so the block's rows are the one range
 // [u0, u0 + 15 + w) (clipped to q_len), walked once per query head, and a
 // slot row keeps every block key of its window (key <= row < key + w)
 // instead of the one key of an entry.
 
-template <int D, Elem E, bool WIN = false>
-__global__ __launch_bounds__(64, 2) void band_dkdv_kernel(BwdArgs A, const float* lse2) {
+template <int D, Elem E, bool WIN, int S>
+__global__ __launch_bounds__(64 * S, 2) void band_dkdv_kernel(BwdArgs A, const float* lse2) {
   using M = MmaT<E>;
   using V8 = typename M::v8;
   using C = BandCfg<D>;
   constexpr int ROWS = 32;                // query rows per step
   constexpr int SLOT2 = ROWS * D;         // elements per Q or dO slot
   constexpr int SL = ROWS * C::CPR / 64;  // DMA instructions per slot
-  __shared__ __attribute__((aligned(1024))) uint16_t qsl[SLOT2];
-  __shared__ __attribute__((aligned(1024))) uint16_t osl[SLOT2];
-  __shared__ __attribute__((aligned(256))) float lsl[64];  // delta, lse2 of the slot rows
+  __shared__ __attribute__((aligned(1024))) uint16_t qsl_[SLOT2 * S];
+  __shared__ __attribute__((aligned(1024))) uint16_t osl_[SLOT2 * S];
+  __shared__ __attribute__((aligned(256))) float lsl_[64 * S];  // delta, lse2 of the slot rows
+  const int wv = S > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
+  uint16_t* const qsl = qsl_ + wv * SLOT2;
+  uint16_t* const osl = osl_ + wv * SLOT2;
+  float* const lsl = lsl_ + 64 * wv;
   lds_u16* const lq = (lds_u16*)qsl;
   lds_u16* const lo = (lds_u16*)osl;
 
@@ -807,7 +816,7 @@ __global__ __launch_bounds__(64, 2) void band_dkdv_kernel(BwdArgs A, const float
   const int kvh = bkv % A.Hkv, b = bkv / A.Hkv;
   const int u0 = 16 * kb;
 
-  const int lane = threadIdx.x;
+  const int lane = S > 1 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
   const int n = lane & 15, q = lane >> 4;
   const int key = u0 + n;
   const bool key_ok = key < A.kv_len;
@@ -928,8 +937,21 @@ __global__ __launch_bounds__(64, 2) void band_dkdv_kernel(BwdArgs A, const float
     s_hi = (int)(steps * (part + 1) / A.split_parts);
   }
 
+  // S waves: each takes whole heads where the group's divide among them, else
+  // its share of every head's (or of the part's) steps
+  const bool by_head = S > 1 && !split && A.groups % S == 0;
+  int hg0 = 0, hg1 = A.groups;
+  if (by_head) {
+    hg0 = A.groups / S * wv;
+    hg1 = hg0 + A.groups / S;
+  }
+  if (S > 1 && split) {
+    const int n = s_hi - s_lo;
+    s_hi = s_lo + (int)((int64_t)n * (wv + 1) / S);
+    s_lo = s_lo + (int)((int64_t)n * wv / S);
+  }
   int s_base = 0;  // steps of the earlier heads
-  for (int hg = 0; hg < A.groups; ++hg) {
+  for (int hg = hg0; hg < hg1; ++hg) {
     const int h = kvh * A.groups + hg;
     const HeadWeights hw = head_weights(A.pc, h);
     auto key_at = [&](int i, int j) {
@@ -939,7 +961,11 @@ __global__ __launch_bounds__(64, 2) void band_dkdv_kernel(BwdArgs A, const float
     int r0, len, cum;
     const int total = head_ranges(h, r0, len, cum);
     const int steps_h = (total + ROWS - 1) / ROWS;
-    const int ls0 = min(max(s_lo - s_base, 0), steps_h), ls1 = min(max(s_hi - s_base, 0), steps_h);
+    int ls0 = min(max(s_lo - s_base, 0), steps_h), ls1 = min(max(s_hi - s_base, 0), steps_h);
+    if (S > 1 && !split && !by_head) {
+      ls0 = steps_h * wv / S;
+      ls1 = steps_h * (wv + 1) / S;
+    }
     s_base += steps_h;
     if (ls0 >= ls1) continue;
     const int p_first = ROWS * ls0, p_end = min(total, ROWS * ls1);
@@ -1115,6 +1141,33 @@ __global__ __launch_bounds__(64, 2) void band_dkdv_kernel(BwdArgs A, const float
     __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
   }
 
+  // ---- S waves: wave w hands its sums to wave 0 through its own slots (16
+  // bytes a lane and slice), which adds them in wave order
+  if constexpr (S > 1) {
+    static_assert(C::NV * 512 <= SLOT2, "a slot holds one accumulator");
+    if (wv > 0) {
+#pragma unroll
+      for (int s = 0; s < C::NV; ++s) {
+        ((f32x4*)qsl)[s * 64 + lane] = dkacc[s];
+        ((f32x4*)osl)[s * 64 + lane] = dvacc[s];
+      }
+    }
+    __syncthreads();
+    if (wv > 0) return;
+#pragma unroll
+    for (int w2 = 1; w2 < S; ++w2)
+#pragma unroll
+      for (int s = 0; s < C::NV; ++s) {
+        const f32x4 x = ((const f32x4*)(qsl_ + w2 * SLOT2))[s * 64 + lane];
+        const f32x4 y = ((const f32x4*)(osl_ + w2 * SLOT2))[s * 64 + lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          dkacc[s][e] += x[e];
+          dvacc[s][e] += y[e];
+        }
+      }
+  }
+
   // ---- a split block: every part stores its float32 sums; the part that
   // arrives last adds the parts in part order (a fixed order whichever wave
   // is last) and writes the block
@@ -1176,22 +1229,63 @@ __global__ __launch_bounds__(64, 2) void band_dkdv_kernel(BwdArgs A, const float
   }
 }
 
+template <int D, Elem E, bool WIN>
+static void launch_band_dkdv_waves(const BwdArgs& a, dim3 grid, int waves, const float* lse2,
+                                   hipStream_t stream) {
+  if (waves == 8)
+    band_dkdv_kernel<D, E, WIN, 8><<<grid, 512, 0, stream>>>(a, lse2);
+  else if (waves == 4)
+    band_dkdv_kernel<D, E, WIN, 4><<<grid, 256, 0, stream>>>(a, lse2);
+  else if (waves == 2)
+    band_dkdv_kernel<D, E, WIN, 2><<<grid, 128, 0, stream>>>(a, lse2);
+  else
+    band_dkdv_kernel<D, E, WIN, 1><<<grid, 64, 0, stream>>>(a, lse2);
+}
+
 template <Elem E>
-static void launch_band_dkdv_elem(const BwdArgs& a, int head_dim, dim3 grid, const float* lse2,
-                                  hipStream_t stream) {
+static void launch_band_dkdv_elem(const BwdArgs& a, int head_dim, dim3 grid, int waves,
+                                  const float* lse2, hipStream_t stream) {
   // a sliding window at interpolation weight 0
   const bool win = a.pc.a == 0.0f;
   if (head_dim == 128) {
     if (win)
-      band_dkdv_kernel<128, E, true><<<grid, 64, 0, stream>>>(a, lse2);
+      launch_band_dkdv_waves<128, E, true>(a, grid, waves, lse2, stream);
     else
-      band_dkdv_kernel<128, E><<<grid, 64, 0, stream>>>(a, lse2);
+      launch_band_dkdv_waves<128, E, false>(a, grid, waves, lse2, stream);
   } else {
     if (win)
-      band_dkdv_kernel<64, E, true><<<grid, 64, 0, stream>>>(a, lse2);
+      launch_band_dkdv_waves<64, E, true>(a, grid, waves, lse2, stream);
     else
-      band_dkdv_kernel<64, E><<<grid, 64, 0, stream>>>(a, lse2);
+      launch_band_dkdv_waves<64, E, false>(a, grid, waves, lse2, stream);
   }
+}
+
+// Waves per key block.  One wave takes a block's whole walk, groups * w steps
+// of 32 rows on average and about ln(kv_len / 16) times that for the first
+// blocks of the last layer (interpolation weight 1), so a grid of few rounds of
+// resident waves (2048 at D = 128, 3072 at D = 64: R rounds) lasts as long as
+// its longest walk.  Two to eight waves share a block there; with more rounds
+// one wave a block is faster (no sums handed over, each head's ranges searched
+// once).  Whole band backward, one wave against the rule's count:
+//   weight 1: H=32/4 L=8192 D=128 (R = 1) 3109 -> 1389 us with 8, H=8/2 L=4096
+//   (R = 0.25) 902 -> 283 with 8, H=8/4 L=8192 (R = 1) 742 -> 412 with 4, B=2
+//   H=8/2 L=16384 (R = 2) 1995 -> 1427 with 4, H=8 L=16384 (R = 4) 722 -> 539
+//   with 2; at R = 6.1 within 1%, at R = 8 and 8 kv heads two waves 8% slower;
+//   weight 4/7: H=8/2 L=4096 367 -> 180 with 4, H=32/4 L=8192 1217 -> 1100, H=4
+//   L=4096 (R = 0.5) 136 -> 119 with 2, H=16/8 L=32768 D=64 (R = 5.3) 1128 ->
+//   1084 with 2; one head a kv head at R = 2 .. 2.7 1-5% slower with 2;
+//   weight 0: H=8/2 L=4096 44 -> 38 with 2; at R = 1 5% slower.
+static int band_dkdv_waves(const BwdArgs& a, int head_dim) {
+  const int resident = head_dim == 128 ? 2048 : 3072;
+  const float R = (float)a.n_kblk / (float)resident;
+  if (a.pc.a == 0.0f) return R <= 0.5f ? 2 : 1;
+  if (a.pc.a == 1.0f) {
+    if (R <= 1.0f) return R <= 0.3f || a.groups >= 4 ? 8 : 4;
+    return R < 4.0f ? 4 : R < 6.0f ? 2 : 1;
+  }
+  if (a.groups >= 4) return R < 4.0f ? 4 : 1;
+  if (R <= 1.0f) return R <= 0.3f ? 4 : 2;
+  return a.groups >= 2 && R < 6.0f ? 2 : 1;
 }
 
 hipError_t launch_band_dkdv(const BwdArgs& a, int head_dim, const float* lse2,
@@ -1209,10 +1303,12 @@ hipError_t launch_band_dkdv(const BwdArgs& a, int head_dim, const float* lse2,
   BwdArgs r = a;
   r.rot_dkdv = band_rotation(a.n_kblk, head_dim == 128 ? 256 : 384,
                              (int64_t)a.q_len * 4 * head_dim, head_dim == 128 ? 19 : 12, 0);
+  const int waves = band_dkdv_waves(a, head_dim);
+  r.rot_dkdv *= waves;  // (a block's walk is that much shorter: 0-4% faster than unscaled)
   if (a.elem == (int)Elem::f16)
-    launch_band_dkdv_elem<Elem::f16>(r, head_dim, grid, lse2, stream);
+    launch_band_dkdv_elem<Elem::f16>(r, head_dim, grid, waves, lse2, stream);
   else
-    launch_band_dkdv_elem<Elem::bf16>(r, head_dim, grid, lse2, stream);
+    launch_band_dkdv_elem<Elem::bf16>(r, head_dim, grid, waves, lse2, stream);
   return hipGetLastError();
 }
 

@@ -1,0 +1,44 @@
+"""The band dK/dV with several waves per key block, at sizes where the rule
+picks 1, 2, 4 and 8: kv groups that divide among the waves and that do not, a
+last key block that is not full, the last layer's split first block
+(groups * q_len > 6144), layer 0's window form, both 16-bit types.
+
+Reference: the block-sparse kernels' dK and dV, which round P and dS to the
+same 16 bits and sum in float32.  Bar: each of a gradient's products carries
+two roundings of 2^-9 (bf16; 2^-12 in f16) and the stored gradients one more
+each; independent over the >= 64 products of a key, at most 4 2^-9 of the
+largest gradient: 8e-3 and 1e-3."""
+import pytest
+import torch
+
+from elastic_sparse_attention import (ElasticSparseAttention, elastic_attention_bwd,
+                                      elastic_attention_fwd)
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda", 0)
+BAR = {torch.bfloat16: 8e-3, torch.float16: 1e-3}
+
+
+@pytest.mark.parametrize("B,H,Hkv,L,D,layer,dtype", [
+    (1, 8, 1, 500, 128, 7, torch.bfloat16), (1, 3, 1, 777, 64, 7, torch.bfloat16),
+    (1, 8, 1, 2000, 64, 7, torch.float16), (2, 4, 2, 8200, 128, 7, torch.bfloat16),
+    (1, 4, 4, 9000, 128, 7, torch.bfloat16), (1, 4, 1, 1003, 128, 3, torch.bfloat16),
+    (1, 6, 2, 1500, 64, 4, torch.bfloat16), (1, 4, 4, 8200, 128, 5, torch.float16),
+    (1, 4, 2, 17000, 64, 2, torch.bfloat16), (1, 2, 2, 150, 128, 4, torch.bfloat16),
+    (1, 6, 2, 333, 128, 0, torch.bfloat16), (1, 4, 1, 16, 64, 0, torch.float16)])
+def test_matches_block_sparse(B, H, Hkv, L, D, layer, dtype):
+    g = torch.Generator(device=DEV).manual_seed(L + H)
+    q, k, v = (torch.randn(B, h, L, D, generator=g, device=DEV, dtype=dtype)
+               for h in (H, Hkv, Hkv))
+    lay = ElasticSparseAttention(layer, 8, H, D, 64, L, num_key_value_heads=Hkv).layout(DEV)
+    o, lse = elastic_attention_fwd(q, k, v, lay, D ** -0.5)
+    go = torch.randn(B, L, H, D, generator=g, device=DEV, dtype=dtype)
+    run = lambda kind: elastic_attention_bwd(q, k, v, o, lse, go, lay, D ** -0.5,  # noqa: E731
+                                             dq_kernel="band", dkdv_kernel=kind)
+    got, ref = run("band"), run("tile")
+    for a, b in zip(got[1:], ref[1:]):
+        err = ((a.float() - b.float()).abs().max() / b.float().abs().max()).item()
+        print(f"  {err:.2e}", flush=True)
+        assert err <= BAR[dtype]
+    again = run("band")
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
