@@ -105,11 +105,11 @@ __all__ = [
 _RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
-def _stream(device: torch.device) -> ctypes.c_void_p:
+def _stream(device: torch.device) -> int:
     if _RAW_STREAM is not None:
-        index = device.index if device.index is not None else torch.cuda.current_device()
-        return ctypes.c_void_p(_RAW_STREAM(index))
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+        index = device.index
+        return _RAW_STREAM(index if index is not None else torch.cuda.current_device())
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 _INITIALISED = set()
@@ -129,15 +129,15 @@ def init_device(device: torch.device) -> None:
     _INITIALISED.add(index)
 
 
+_DTYPE_CODES = {torch.bfloat16: ESA_BF16, torch.float32: ESA_F32, torch.float16: ESA_F16}
+
+
 def _dtype_code(dt: torch.dtype) -> int:
-    if dt == torch.bfloat16:
-        return ESA_BF16
-    if dt == torch.float32:
-        return ESA_F32
-    if dt == torch.float16:
-        return ESA_F16
-    raise ValueError(f"unsupported dtype {dt}: the HIP kernels take bfloat16, float16 or "
-                     "float32")
+    code = _DTYPE_CODES.get(dt)
+    if code is None:
+        raise ValueError(f"unsupported dtype {dt}: the HIP kernels take bfloat16, float16 or "
+                         "float32")
+    return code
 
 
 def _require_gpu(*ts: torch.Tensor) -> None:
@@ -149,12 +149,19 @@ def _require_gpu(*ts: torch.Tensor) -> None:
 
 
 def _prep(t: torch.Tensor, align_elems: int) -> torch.Tensor:
-    """Innermost dim contiguous, base and strides aligned for row loads."""
+    """Innermost dim contiguous, base and strides aligned for row loads (to
+    ``align_elems`` elements, a power of two)."""
+    st = t.stride()
+    low = align_elems - 1
     es = t.element_size()
-    ok = (t.stride(-1) == 1 and t.data_ptr() % (align_elems * es) == 0
-          and all(s % align_elems == 0 for s in t.stride()[:-1]))
-    if ok:
-        return t
+    # (one bit test for all strides and one for the base: a decode step pays
+    # for these per call)
+    if st[-1] == 1 and t.data_ptr() % (align_elems * es) == 0:
+        bits = 0
+        for x in st[:-1]:
+            bits |= x
+        if bits & low == 0:
+            return t
     t = t.contiguous()
     if t.data_ptr() % (align_elems * es) != 0:
         t = t.clone()
@@ -438,41 +445,37 @@ def _fwd_args(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor
               o_strides: Tuple[int, int, int], lse: Optional[torch.Tensor],
               scaling: float) -> EsaFwdArgs:
     B, H, Lq, D = q.shape
-    a = EsaFwdArgs()
-    a.dtype = _dtype_code(q.dtype)
-    a.batch, a.num_heads, a.num_kv_heads = B, H, k.shape[1]
-    a.q_len, a.kv_len, a.head_dim = Lq, k.shape[2], D
-    a.q = q.data_ptr()
-    a.q_stride_b, a.q_stride_h, a.q_stride_s = q.stride()[:3]
-    a.k = k.data_ptr()
-    a.k_stride_b, a.k_stride_h, a.k_stride_s = k.stride()[:3]
-    a.v = v.data_ptr()
-    a.v_stride_b, a.v_stride_h, a.v_stride_s = v.stride()[:3]
-    a.o = o.data_ptr()
-    a.o_stride_b, a.o_stride_h, a.o_stride_s = o_strides
+    _, Hkv, Lk, _ = k.shape
+    qs, ks, vs = q.stride(), k.stride(), v.stride()
     if lse is not None:
-        a.lse = lse.data_ptr()
-        a.lse_stride_b, a.lse_stride_h = lse.stride(0), lse.stride(1)
+        ls = lse.stride()
+        lp, lb, lh = lse.data_ptr(), ls[0], ls[1]
     else:
-        a.lse = None
-    a.sm_scale = float(scaling)
-    return a
+        lp, lb, lh = None, 0, 0
+    # in the order of esa_fwd_args' fields
+    return EsaFwdArgs(_dtype_code(q.dtype), B, H, Hkv, Lq, Lk, D,
+                      q.data_ptr(), qs[0], qs[1], qs[2], k.data_ptr(), ks[0], ks[1], ks[2],
+                      v.data_ptr(), vs[0], vs[1], vs[2], o.data_ptr(), *o_strides,
+                      lp, lb, lh, float(scaling))
 
 
 def _check_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
-    _require_gpu(q, k, v)
-    if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
+    if not (q.is_cuda and k.is_cuda and v.is_cuda):
+        _require_gpu(q, k, v)
+    qs, ks, vs = q.shape, k.shape, v.shape
+    if len(qs) != 4 or len(ks) != 4 or len(vs) != 4:
         raise ValueError("q, k, v must be 4-D [B, heads, seq, head_dim]")
-    if k.shape != v.shape:
-        raise ValueError(f"key {tuple(k.shape)} and value {tuple(v.shape)} shapes differ")
-    if q.shape[0] != k.shape[0] or q.shape[3] != k.shape[3]:
-        raise ValueError(f"query {tuple(q.shape)} and key {tuple(k.shape)} disagree on batch "
+    if ks != vs:
+        raise ValueError(f"key {tuple(ks)} and value {tuple(vs)} shapes differ")
+    if qs[0] != ks[0] or qs[3] != ks[3]:
+        raise ValueError(f"query {tuple(qs)} and key {tuple(ks)} disagree on batch "
                          "or head_dim")
-    if q.dtype != k.dtype or q.dtype != v.dtype:
+    dt = q.dtype
+    if dt != k.dtype or dt != v.dtype:
         raise ValueError("q, k and v must share one dtype")
-    if q.shape[1] % k.shape[1] != 0:
-        raise ValueError(f"query heads ({q.shape[1]}) must be divisible by key/value heads "
-                         f"({k.shape[1]})")
+    if qs[1] % ks[1] != 0:
+        raise ValueError(f"query heads ({qs[1]}) must be divisible by key/value heads "
+                         f"({ks[1]})")
 
 
 # input types the MFMA prefill kernels take (others run the per-row gather)
@@ -765,7 +768,7 @@ def _positions_ptr(positions: Optional[torch.Tensor], q_len: int, device: torch.
             positions.numel() != q_len:
         raise ValueError("positions must be an int64 tensor of q_len entries on q's device")
     positions = positions.contiguous()
-    return positions, ctypes.c_void_p(positions.data_ptr())
+    return positions, positions.data_ptr()
 
 
 def elastic_attention_rows(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
@@ -792,11 +795,12 @@ def _rows_fwd(q, k, v, pattern, scaling, positions, return_lse, dropout_p, seed,
     """elastic_attention_rows after its argument checks (the module, which
     checks q, k, v itself, calls this directly)."""
     B, H, Lq, D = q.shape
+    device = q.device
     q, k, v = _prep(q, 4), _prep(k, 4), _prep(v, 4)
-    o = torch.empty(B, Lq, H, D, dtype=q.dtype, device=q.device)
+    o = torch.empty((B, Lq, H, D), dtype=q.dtype, device=device)
     need_lse = return_lse or return_weights
-    lse = torch.empty(B, H, Lq, dtype=torch.float32, device=q.device) if need_lse else None
-    positions, pos_ptr = _positions_ptr(positions, Lq, q.device)
+    lse = torch.empty(B, H, Lq, dtype=torch.float32, device=device) if need_lse else None
+    positions, pos_ptr = _positions_ptr(positions, Lq, device)
     if B == 0 or Lq == 0:
         lse_out = lse if return_lse else None
         if return_weights:
@@ -804,7 +808,7 @@ def _rows_fwd(q, k, v, pattern, scaling, positions, return_lse, dropout_p, seed,
                               device=q.device)
             return o, lse_out, wts
         return o, lse_out
-    a = _fwd_args(q, k, v, o, (o.stride(0), o.stride(2), o.stride(1)), lse, scaling)
+    a = _fwd_args(q, k, v, o, (Lq * H * D, D, H * D), lse, scaling)  # (o is contiguous)
     if dropout_p > 0.0 or return_weights:
         wts = None
         opts = EsaNaiveOpts()
@@ -815,12 +819,12 @@ def _rows_fwd(q, k, v, pattern, scaling, positions, return_lse, dropout_p, seed,
             opts.weights = wts.data_ptr()
             opts.weights_stride_b, opts.weights_stride_h, opts.weights_stride_s = wts.stride()[:3]
         check(load().esa_elastic_fwd_naive(ctypes.byref(a), ctypes.byref(pattern), pos_ptr,
-                                           ctypes.byref(opts), _stream(q.device)),
+                                           ctypes.byref(opts), _stream(device)),
               "esa_elastic_fwd_naive")
         lse_out = lse if return_lse else None
         return (o, lse_out, wts) if return_weights else (o, lse_out)
     check(load().esa_elastic_fwd_rows(ctypes.byref(a), ctypes.byref(pattern), pos_ptr,
-                                      _stream(q.device)), "esa_elastic_fwd_rows")
+                                      _stream(device)), "esa_elastic_fwd_rows")
     return o, lse
 
 
@@ -1290,7 +1294,7 @@ class ElasticSparseAttention(nn.Module):
         waits on the GPU: the kernel writes NaN for a row whose position is
         out of range."""
         if isinstance(cache_position, torch.Tensor) and cache_position.is_cuda:
-            pos = cache_position.reshape(-1)
+            pos = cache_position if cache_position.dim() == 1 else cache_position.reshape(-1)
             if pos.dtype != torch.int64 or not pos.is_contiguous():
                 pos = pos.to(torch.int64).contiguous()
             if pos.numel() != q_len:
@@ -1363,6 +1367,18 @@ class ElasticSparseAttention(nn.Module):
             o, _ = elastic_attention_band(q, k, v, self.pattern, self.scaling, return_lse=False,
                                           positions=pos)
             return o.view(B, Lq, H * D), None                              # :761-763
+        if not grad and not naive and dropout_p == 0.0:
+            # per-row gather without weights or dropout (a decode step): into
+            # an output of the module's own shape, with pos as checked above
+            q, k, v = _prep(q, 4), _prep(k, 4), _prep(v, 4)
+            device = q.device
+            o = torch.empty((B, Lq, H * D), dtype=q.dtype, device=device)
+            if B > 0 and Lq > 0:
+                a = _fwd_args(q, k, v, o, (Lq * H * D, D, H * D), None, self.scaling)
+                check(load().esa_elastic_fwd_rows(ctypes.byref(a), ctypes.byref(self.pattern),
+                                                  None if pos is None else pos.data_ptr(),
+                                                  _stream(device)), "esa_elastic_fwd_rows")
+            return o, None
         # per-row gather: decode rows, float32 / float16, other head dims, the
         # naive path; keep decisions of dropout drawn from torch's generator
         seed = int(torch.randint(0, 1 << 62, (1,)).item()) if dropout_p > 0.0 else 0
