@@ -764,7 +764,10 @@ __global__ __launch_bounds__(64, 2) void window_dq_kernel(BwdArgs A, const float
 //
 // WIN: interpolation weight 0 (layer 0, a sliding window).  Key u is
 // attended by rows u .. u + w - 1, so the block's rows are the one range
-// [u0, u0 + 15 + w) (clipped to q_len), walked once per query head, and a
+// [u0, u0 + 15 + w) (clipped to q_len), walked once per query head (the heads'
+// steps as one sequence, the next head's first rows in flight during a head's
+// last step: H=32/8 L=32768 D=128 backward 608 -> 591 us with the heads' step
+// counts known, H=32/4 L=8192 146 -> 135, H=16/4 B=8 L=4096 D=64 154 -> 143), and a
 // slot row keeps every block key of its window (key <= row < key + w)
 // instead of the one key of an entry.
 
@@ -897,10 +900,7 @@ __global__ __launch_bounds__(64 * S, 2) void band_dkdv_kernel(BwdArgs A, const f
     r0 = 0;
     len = 0;
     const int ej = (lane + rot) & 63;
-    if constexpr (WIN) {
-      r0 = u0;
-      len = lane == 0 ? max(min(u0 + 15 + A.pc.w, A.q_len) - u0, 0) : 0;
-    } else if (ej < A.pc.w) {
+    if (ej < A.pc.w) {
       int a0 = u0, a1 = A.q_len;  // first row >= u0 with key >= u0
       while (a0 < a1) {
         const int mid = (a0 + a1) >> 1;
@@ -939,7 +939,7 @@ __global__ __launch_bounds__(64 * S, 2) void band_dkdv_kernel(BwdArgs A, const f
 
   // S waves: each takes whole heads where the group's divide among them, else
   // its share of every head's (or of the part's) steps
-  const bool by_head = S > 1 && !split && A.groups % S == 0;
+  const bool by_head = !WIN && S > 1 && !split && A.groups % S == 0;
   int hg0 = 0, hg1 = A.groups;
   if (by_head) {
     hg0 = A.groups / S * wv;
@@ -950,16 +950,25 @@ __global__ __launch_bounds__(64 * S, 2) void band_dkdv_kernel(BwdArgs A, const f
     s_hi = s_lo + (int)((int64_t)n * (wv + 1) / S);
     s_lo = s_lo + (int)((int64_t)n * wv / S);
   }
+  // WIN: every head has the same steps, and the heads' steps run as one
+  // sequence (each wave a share of it), so the next head's first rows are
+  // requested during this head's last step
+  const int win_rows = max(min(u0 + 15 + A.pc.w, A.q_len) - u0, 0);
+  const int win_steps = max((win_rows + ROWS - 1) / ROWS, 1);
+  if constexpr (WIN) hg1 = 1;
   int s_base = 0;  // steps of the earlier heads
   for (int hg = hg0; hg < hg1; ++hg) {
-    const int h = kvh * A.groups + hg;
+    int h = kvh * A.groups + hg;
     const HeadWeights hw = head_weights(A.pc, h);
     auto key_at = [&](int i, int j) {
       const RowParams rp = row_params(A.pc, i);
       return interp_index(oversized(rp, j), oversized(rp, j + 1), hw);
     };
-    int r0, len, cum;
-    const int total = head_ranges(h, r0, len, cum);
+    int r0 = 0, len = 0, cum = 0, total;
+    if constexpr (WIN)
+      total = win_rows > 0 ? A.groups * win_steps * ROWS : 0;
+    else
+      total = head_ranges(h, r0, len, cum);
     const int steps_h = (total + ROWS - 1) / ROWS;
     int ls0 = min(max(s_lo - s_base, 0), steps_h), ls1 = min(max(s_hi - s_base, 0), steps_h);
     if (S > 1 && !split && !by_head) {
@@ -977,6 +986,11 @@ __global__ __launch_bounds__(64 * S, 2) void band_dkdv_kernel(BwdArgs A, const f
     auto map_step = [&](int P, int& e, int& row, int& ent) {
       row = -1;
       ent = 0;
+      if constexpr (WIN) {
+        const int d = P % (win_steps * ROWS) + slot_row;
+        row = d < win_rows ? u0 + d : -1;
+        return;
+      }
       while (e < 64) {
         const int ce = __builtin_amdgcn_readlane(cum, e);
         if (ce >= P + ROWS) break;
@@ -993,16 +1007,22 @@ __global__ __launch_bounds__(64 * S, 2) void band_dkdv_kernel(BwdArgs A, const f
       }
     };
 
-    const char* const qbase = (const char*)(A.q + (int64_t)b * A.qsb + (int64_t)h * A.qsh);
-    const char* const obase = (const char*)(A.dout + (int64_t)b * A.dosb + (int64_t)h * A.dosh);
-    const char* const sbase = (const char*)(A.delta + ((int64_t)b * A.H + h) * A.qpad);
-    const __amdgpu_buffer_rsrc_t qrs =
-        __builtin_amdgcn_make_buffer_rsrc((void*)qbase, (short)0, A.q_len * qss2, 0x00020000);
-    const __amdgpu_buffer_rsrc_t ors =
-        __builtin_amdgcn_make_buffer_rsrc((void*)obase, (short)0, A.q_len * oss2, 0x00020000);
-    // delta row of (b, h) and, lse_off bytes further, its lse2 row
-    const __amdgpu_buffer_rsrc_t srs = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)sbase, (short)0, lse_off + 4 * A.qpad, 0x00020000);
+    __amdgpu_buffer_rsrc_t qrs, ors, srs;
+    // head h's Q and dO rows; its delta row and, lse_off bytes further, its
+    // lse2 row
+    auto set_head = [&](int h) {
+      qrs = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(A.q + (int64_t)b * A.qsb + (int64_t)h * A.qsh), (short)0, A.q_len * qss2,
+          0x00020000);
+      ors = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(A.dout + (int64_t)b * A.dosb + (int64_t)h * A.dosh), (short)0, A.q_len * oss2,
+          0x00020000);
+      srs = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(A.delta + ((int64_t)b * A.H + h) * A.qpad), (short)0, lse_off + 4 * A.qpad,
+          0x00020000);
+    };
+    if constexpr (WIN) h = kvh * A.groups + p_first / (win_steps * ROWS);
+    set_head(h);
     // Q or dO rows of the step whose slot rows hold `row` -> slot dst (after
     // the step's reads of dst)
     auto issue_rows = [&](__amdgpu_buffer_rsrc_t rs, int ss2, int row, lds_u16* dst) {
@@ -1028,7 +1048,8 @@ __global__ __launch_bounds__(64 * S, 2) void band_dkdv_kernel(BwdArgs A, const f
     };
 
     // the first live entry reaching past the part's first position
-    int e = (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(len > 0 && cum + len > p_first));
+    int e = WIN ? 0
+                : (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(len > 0 && cum + len > p_first));
     int row_c, ent_c;
     map_step(p_first, e, row_c, ent_c);
     issue_rows(qrs, qss2, row_c, lq);
@@ -1037,7 +1058,13 @@ __global__ __launch_bounds__(64 * S, 2) void band_dkdv_kernel(BwdArgs A, const f
     issue_stats(row_c);
     for (int P = p_first; P < p_end; P += ROWS) {
       int row_n = -1, ent_n = 0;
-      if (P + ROWS < p_end) map_step(P + ROWS, e, row_n, ent_n);
+      if (P + ROWS < p_end) {
+        map_step(P + ROWS, e, row_n, ent_n);
+        if constexpr (WIN) {
+          const int hn = kvh * A.groups + (P + ROWS) / (win_steps * ROWS);
+          if (hn != h) set_head(h = hn);
+        }
+      }
       // the key of slot row (lane % 32), -1 when masked or empty
       int rkey = -1;
       if constexpr (WIN) {
