@@ -785,6 +785,9 @@ bool coop_applies(GatherBwdArgs& a, int es) {
   a.q_span = (int)qs;
   a.do_span = (int)gs;
   const int64_t rows = (int64_t)a.H * a.q_len;
+  // (64 work-items a row and a key, 2^32 a grid dimension)
+  constexpr int64_t kMost = (int64_t(1) << 26) - 64;
+  if (rows > kMost || (int64_t)a.Hkv * a.kv_len > kMost) return false;
   // the per-entry coefficients' 2 B E floats hold the rows' (lse, delta) and
   // the partial sums of long segments, in windows of at least 512 entries
   a.ld2 = (float2*)a.cp;

@@ -420,7 +420,8 @@ esa_status esa_elastic_bwd(const esa_bwd_args* a, const esa_pattern* p,
 
 /* Host only.  Bytes of workspace esa_sparse_bwd and esa_elastic_bwd_rows
  * need for index lists of attn_length entries per row: per batch element and
- * entry two float32 coefficients, four uint32 arrays of entries for the sort,
+ * entry two float32 words (coefficients, or the rows' lse and delta and partial
+ * sums), four uint32 arrays of entries for the sort,
  * (num_kv_heads * kv_len + 1) int32 segment starts, and the sort's
  * histograms (each region 256-byte aligned).  Requires num_heads * q_len *
  * attn_length and num_kv_heads * kv_len below 2^31 - 1. */
@@ -435,10 +436,10 @@ esa_status esa_gather_bwd_workspace_size(const esa_bwd_args* a, int32_t attn_len
  * reaches get 0, as the reference's zeros_like does).  Semantics of the
  * reference: p = exp(scale q.k - lse) on valid entries; an entry whose index
  * lies outside [0, kv_len) scores 0 against zero K/V and adds nothing to dk or
- * dv; an entry listed twice counts twice.  No atomics on the gradients: each
- * entry's dK / dV coefficients go to the workspace, a stable radix sort
- * groups them by key, and one wave sums each key's entries in entry order,
- * so results are deterministic.  dtype ESA_F32, ESA_BF16 or ESA_F16
+ * dv; an entry listed twice counts twice.  No atomics on the gradients: a
+ * stable radix sort groups the entries by key, and each key's entries are
+ * summed in entry order by one wave (long lists in windows, the windows in
+ * order), so results are deterministic.  dtype ESA_F32, ESA_BF16 or ESA_F16
  * (float32 arithmetic), head_dim a multiple of 4 up to 256, K / V rows
  * aligned to 4 elements; workspace from esa_gather_bwd_workspace_size,
  * 256-byte aligned. */
