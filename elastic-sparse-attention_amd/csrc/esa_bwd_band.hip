@@ -53,7 +53,7 @@ __global__ __launch_bounds__(64, 2) void band_dq_kernel(BwdArgs A, const float* 
   const int bid = blockIdx.x;
   const int g = (bid & 7) * A.per_xcd + (bid >> 3);
   if (g >= A.n_groups) return;
-  const GroupId id = group_id(g, A.ng, 1, A.H, A.groups);
+  const GroupId id = group_id(g, A.order);
   const int b = id.b, h = id.h, kvh = id.kvh, gq = id.gq;
 
   const int lane = threadIdx.x;
@@ -457,7 +457,7 @@ __global__ __launch_bounds__(64, 2) void window_dq_kernel(BwdArgs A, const float
   const int bid = blockIdx.x;
   const int g = (bid & 7) * per2 + (bid >> 3);
   if (g >= n2) return;
-  const GroupId id = group_id(g, ng2, A.win_inner, A.H, A.groups);
+  const GroupId id = group_id(g, A.order);
   const int b = id.b, h = id.h, kvh = id.kvh, gq = id.gq;
 
   const int lane = threadIdx.x;
@@ -1350,7 +1350,8 @@ static void launch_band_dq_d(const BwdArgs& a, dim3 grid, const float* lse2, hip
     // L2 (group_id): B=1 H=32/8 L=32768 D=128 backward 642 -> 608 us, H=32/4
     // L=8192 150 -> 146; below that 0-2% slower (B=8 H=16/4 L=4096 D=64 153 -> 157)
     BwdArgs w = a;
-    w.win_inner = (int64_t)a.kv_len * 4 * D >= (int64_t(4) << 20) ? a.groups : 1;
+    const int inner = (int64_t)a.kv_len * 4 * D >= (int64_t(4) << 20) ? a.groups : 1;
+    w.order = make_group_order((a.q_len + 31) / 32, inner, a.H, a.groups);
     window_dq_kernel<D, PREP, E><<<dim3((unsigned)(8 * ((n2 + 7) / 8))), 64, 0, stream>>>(w, lse2);
   } else if (a.pc.a >= 0.5f)
     band_dq_kernel<D, true, PREP, E><<<grid, 64, 0, stream>>>(a, lse2);
@@ -1385,6 +1386,7 @@ hipError_t launch_band_dq(const BwdArgs& a, int head_dim, const float* lse2, boo
   // 12/64); none for a grid of a few rounds whose heads' K and V exceed L2
   // (band_rotation, measured with the dK / dV's in launch_band_dkdv)
   BwdArgs r = a;
+  r.order = make_group_order(a.ng, 1, a.H, a.groups);
   r.rot_dq = band_rotation(a.n_groups, head_dim == 128 ? 256 : 512,
                            (int64_t)a.kv_len * 4 * head_dim, head_dim == 128 ? 19 : 12, 0);
   if (a.elem == (int)Elem::f16)

@@ -94,7 +94,7 @@ __global__ __launch_bounds__(64 * S, 2) void band_fwd_kernel(BandArgs A) {
   const int bid = blockIdx.x;
   const int g = (bid & 7) * A.per_xcd + (bid >> 3);
   if (g >= A.n_groups) return;
-  const GroupId id = group_id(g, A.ng, A.inner, A.H, A.groups);
+  const GroupId id = group_id(g, A.order);
   const int b = id.b, h = id.h, kvh = id.kvh, gq = id.gq;
 
   const int lane = S > 1 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
@@ -762,7 +762,8 @@ hipError_t launch_band_fwd(const BandArgs& a, int head_dim, hipStream_t stream) 
   // 8192 rows 633 -> 511; early chunks and D=64 within 2%.  At layer 2 of
   // L=100000 16384 rows were 7% slower with a limit of 16 rounds, and H=32/16
   // there 11-15%.  Full prefills of few heads: between -7% (layer 1) and +2%.
-  r.inner = a.positions && r.rot_rate == 3 ? a.groups : 1;
+  const int inner = a.positions && r.rot_rate == 3 ? a.groups : 1;
+  r.order = make_group_order(a.ng, inner, a.H, a.groups);
   // K DMA skipping: with the late V order from interpolation weight 1/2 on
   // (measured at B=1, H=32, L=32768, D=128, w=64 over 8 layers: 1-7% faster
   // at weights 4/7 .. 1, even at 3/7, 3-4% slower at 1/7 and 2/7, where

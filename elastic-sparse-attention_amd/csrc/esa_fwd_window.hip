@@ -63,7 +63,7 @@ __global__ __launch_bounds__(64, 2) void window_fwd_kernel(BandArgs A) {
   if (g >= A.n_groups) return;
   // (the query heads of a kv group together: they list the same keys; H=32/4
   // L=8192 D=128 49.0 -> 45.7 us, H=16/8 B=2 L=16384 D=64 45.6 -> 44.4)
-  const GroupId id = group_id(g, A.ng, A.groups, A.H, A.groups);
+  const GroupId id = group_id(g, A.order);
   const int b = id.b, h = id.h, kvh = id.kvh, gq = id.gq;
 
   const int lane = threadIdx.x;
@@ -375,6 +375,7 @@ void launch_window_d(const BandArgs& a, hipStream_t stream) {
   const int64_t n = (int64_t)a.n_groups / a.ng * w.ng;  // batch * H * ng
   w.n_groups = (int)n;
   w.per_xcd = (int)((n + 7) / 8);
+  w.order = make_group_order(w.ng, a.groups, a.H, a.groups);
   const dim3 grid((unsigned)(8 * w.per_xcd));
   if (a.positions)
     window_fwd_kernel<D, WINDOW_G, E, true><<<grid, 64, 0, stream>>>(w);

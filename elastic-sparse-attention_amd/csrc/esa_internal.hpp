@@ -40,6 +40,38 @@ struct TileArgs {
   const uint32_t* smask;
 };
 
+// Division of n < 2^31 by a fixed d >= 1: n / d = (n * mul) >> shift, with
+// mul = floor(2^(31 + s) / d) + 1, s = ceil(log2 d) (Granlund and Montgomery,
+// "Division by invariant integers using multiplication", PLDI 1994):
+// mul * d - 2^(31 + s) is in 1 .. 2^s, so the error n * that / (2^(31 + s) d)
+// stays below 1 / d.
+struct FastDiv {
+  uint32_t mul;
+  int shift;
+};
+inline FastDiv make_fast_div(uint32_t d) {
+  int s = 0;
+  while ((uint64_t(1) << s) < d) ++s;
+  return FastDiv{(uint32_t)((uint64_t(1) << (31 + s)) / d + 1), 31 + s};
+}
+__host__ __device__ inline uint32_t fast_div(uint32_t n, const FastDiv& f) {
+  return (uint32_t)(((uint64_t)n * f.mul) >> f.shift);
+}
+
+// The order in which a grid takes the 16-row (or 32-row) groups of every
+// (batch, head), see group_id: ng groups a head, `inner` query heads run
+// together (1, or the query heads that share a K and V).
+struct GroupOrder {
+  FastDiv per, inner, outer, groups;
+  int n_per, n_inner, n_outer;
+};
+inline GroupOrder make_group_order(int ng, int inner, int H, int groups) {
+  const int per = ng * inner, outer = H / inner;
+  return GroupOrder{make_fast_div((uint32_t)per), make_fast_div((uint32_t)inner),
+                    make_fast_div((uint32_t)outer), make_fast_div((uint32_t)groups), per, inner,
+                    outer};
+}
+
 // Arguments of the band-gathered forward (prefill rows 0 .. q_len - 1).
 struct BandArgs {
   const uint16_t* q;
@@ -68,9 +100,10 @@ struct BandArgs {
   // dims d_real .. D - 1 of Q, K and V read as zeros and O's are not stored
   int d_real;
   // entry rotation of the band forward, in 64ths of an entry per group
-  // dispatched on an XCD, and the query heads run together (group_id; both set
-  // by launch_band_fwd from the grid's size)
-  int rot_rate, inner;
+  // dispatched on an XCD, and the order of its groups (both set by
+  // launch_band_fwd from the grid's size)
+  int rot_rate;
+  GroupOrder order;
 };
 
 // Where a query row's w entries come from: the elastic pattern (regenerated
@@ -123,24 +156,6 @@ struct GatherArgs {
   int k_span, v_span;
   int waves, waves_per_xcd;
 };
-
-// Division of n < 2^31 by a fixed d >= 1: n / d = (n * mul) >> shift, with
-// mul = floor(2^(31 + s) / d) + 1, s = ceil(log2 d) (Granlund and Montgomery,
-// "Division by invariant integers using multiplication", PLDI 1994):
-// mul * d - 2^(31 + s) is in 1 .. 2^s, so the error n * that / (2^(31 + s) d)
-// stays below 1 / d.
-struct FastDiv {
-  uint32_t mul;
-  int shift;
-};
-inline FastDiv make_fast_div(uint32_t d) {
-  int s = 0;
-  while ((uint64_t(1) << s) < d) ++s;
-  return FastDiv{(uint32_t)((uint64_t(1) << (31 + s)) / d + 1), 31 + s};
-}
-__host__ __device__ inline uint32_t fast_div(uint32_t n, const FastDiv& f) {
-  return (uint32_t)(((uint64_t)n * f.mul) >> f.shift);
-}
 
 // Arguments of the gather backward (any index source, float32 / bfloat16 /
 // float16): per-row pass (dQ and each entry's dK / dV coefficients), a stable
@@ -251,8 +266,8 @@ struct BwdArgs {
   // entry rotation of the band dQ / dK-dV walks, in 64ths of an entry per
   // group or block dispatched on an XCD (set by their launchers)
   int rot_dq, rot_dkdv;
-  // query heads the window dQ runs together (group_id; set by its launcher)
-  int win_inner;
+  // order of the band or window dQ's groups (set by their launcher)
+  GroupOrder order;
 };
 
 // Entry rotation rate of a band kernel's launch (64ths of an entry per unit

@@ -24,7 +24,8 @@ def make(B, H, Hkv, Lq, L, D, dtype):
 @pytest.mark.parametrize("B,H,Hkv,L,D,dtype", [(2, 8, 2, 333, 64, torch.bfloat16),
                                                (1, 6, 2, 1000, 128, torch.float16),
                                                (1, 4, 1, 8200, 128, torch.bfloat16),
-                                               (1, 2, 1, 31, 64, torch.bfloat16)])
+                                               (1, 2, 1, 31, 64, torch.bfloat16),
+                                               (3, 21, 3, 1043, 64, torch.bfloat16)])
 def test_window_kernels(B, H, Hkv, L, D, dtype):
     q, k, v, kr, vr = make(B, H, Hkv, L, L, D, dtype)
     a = ElasticSparseAttention(0, 8, H, D, 64, L, num_key_value_heads=Hkv).layout(DEV)
@@ -40,7 +41,8 @@ def test_window_kernels(B, H, Hkv, L, D, dtype):
 @pytest.mark.parametrize("H,Hkv,L,rows,D,layer", [(8, 2, 20000, 1003, 128, 4),
                                                   (8, 1, 9000, 3000, 128, 2),
                                                   (6, 3, 40000, 500, 64, 7),
-                                                  (32, 4, 12000, 7000, 128, 7)])
+                                                  (32, 4, 12000, 7000, 128, 7),
+                                                  (21, 3, 9001, 2999, 128, 5)])
 def test_chunks(H, Hkv, L, rows, D, layer):
     q, k, v, kr, vr = make(1, H, Hkv, rows, L, D, torch.bfloat16)
     pos = torch.arange(L - rows, L, device=DEV)
