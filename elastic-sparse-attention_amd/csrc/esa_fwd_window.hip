@@ -61,8 +61,6 @@ __global__ __launch_bounds__(64, 2) void window_fwd_kernel(BandArgs A) {
   const int bid = blockIdx.x;
   const int g = (bid & 7) * A.per_xcd + (bid >> 3);
   if (g >= A.n_groups) return;
-  // (the query heads of a kv group together: they list the same keys; H=32/4
-  // L=8192 D=128 49.0 -> 45.7 us, H=16/8 B=2 L=16384 D=64 45.6 -> 44.4)
   const GroupId id = group_id(g, A.order);
   const int b = id.b, h = id.h, kvh = id.kvh, gq = id.gq;
 
@@ -375,7 +373,18 @@ void launch_window_d(const BandArgs& a, hipStream_t stream) {
   const int64_t n = (int64_t)a.n_groups / a.ng * w.ng;  // batch * H * ng
   w.n_groups = (int)n;
   w.per_xcd = (int)((n + 7) / 8);
-  w.order = make_group_order(w.ng, a.groups, a.H, a.groups);
+  // The query heads of a kv group together: they list the same keys.  Prefills
+  // over inputs that change (K and V not left in a cache by the last call)
+  // H=32/8 L=32768 D=128 231 -> 213 us, H=16/8 L=65536 242 -> 218, H=32/4 L=8192
+  // 56 -> 52, H=32/8 L=32768 D=64 109 -> 104; 64 sampled prefills between -5%
+  // and +12%, 2% faster on average.  Not in chunks whose kv heads fill the
+  // XCDs (8 or more): from one to five rounds of resident waves (256 an XCD at
+  // D = 128) they ran 2-8% slower together (the last 3000 rows of H=32/8
+  // L=32768 22.7 -> 24.6 us, 6000 rows at D=64 20.7 -> 21.7, whatever the
+  // length), below that within 1%; above it (16384 rows) 1-7% faster.
+  const int n_kv = a.n_groups / a.ng / a.groups;  // batch * kv heads
+  const bool in_turn = a.positions && n_kv >= 8 && w.per_xcd <= 163840 / D;
+  w.order = make_group_order(w.ng, in_turn ? 1 : a.groups, a.H, a.groups);
   const dim3 grid((unsigned)(8 * w.per_xcd));
   if (a.positions)
     window_fwd_kernel<D, WINDOW_G, E, true><<<grid, 64, 0, stream>>>(w);
