@@ -761,8 +761,16 @@ hipError_t launch_band_fwd(const BandArgs& a, int head_dim, hipStream_t stream) 
   // 1003 -> 616 / 654; H=32/8 L=100000 8192 rows 753 -> 354; H=32/16 L=65536
   // 8192 rows 633 -> 511; early chunks and D=64 within 2%.  At layer 2 of
   // L=100000 16384 rows were 7% slower with a limit of 16 rounds, and H=32/16
-  // there 11-15%.  Full prefills of few heads: between -7% (layer 1) and +2%.
-  const int inner = a.positions && r.rot_rate == 3 ? a.groups : 1;
+  // there 11-15%.  Full prefills take the heads in turn: together they were
+  // between 7% faster (H=2, layer 1) and 24% slower (H=8/2 L=131072 layer 4,
+  // whose rotation is tuned to one head).
+  // Not where an XCD's range holds two heads or more and under 96 groups: all
+  // of them run at once, and their waves' starts spread over the heads cost
+  // less than the keys' rows shared (H=16/2 L=65000 D=128 327 rows, layers 5
+  // and 7 of 8 and 20 of 24 20.0 / 25.0 / 20.0 -> 19.5 / 24.4 / 19.1 us; at 126
+  // groups an XCD, 1000 rows, 29.7 in turn against 25.9).
+  const bool at_once = a.per_xcd < 96 && a.n_groups >= 16 * a.ng;
+  const int inner = a.positions && r.rot_rate == 3 && !at_once ? a.groups : 1;
   r.order = make_group_order(a.ng, inner, a.H, a.groups);
   // K DMA skipping: with the late V order from interpolation weight 1/2 on
   // (measured at B=1, H=32, L=32768, D=128, w=64 over 8 layers: 1-7% faster
