@@ -4,6 +4,8 @@ by `groups` query heads against the same call with K and V repeated per query
 head (groups = 1, the heads one after another).  Sizes: a last row group that
 is not full, group counts that leave the last XCD short, chunks whose grids
 take the few-round rule (a head's K and V above 4 MB), the window kernels."""
+import time
+
 import pytest
 import torch
 
@@ -53,3 +55,34 @@ def test_chunks(H, Hkv, L, rows, D, layer):
     # another entry: equal up to float32 sums and one rounding to bf16
     assert (lse - lse1).abs().max().item() <= 1e-5
     assert (o.float() - o1.float()).abs().max().item() <= 2.0 ** -7 * o.float().abs().max().item()
+
+
+def times(calls, rounds=12, n=40):
+    """Seconds a call of each, the best of `rounds` blocks taken in turn."""
+    best = [float("inf")] * len(calls)
+    for f in calls:
+        f()
+    for _ in range(rounds):
+        for i, f in enumerate(calls):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(n):
+                f()
+            torch.cuda.synchronize()
+            best[i] = min(best[i], (time.perf_counter() - t0) / n)
+    return best
+
+
+def test_shared_heads_cost_no_time():
+    """A chunk of the sliding-window layer over shared kv heads takes no longer
+    than over the same K and V repeated per query head, which reads `groups`
+    times the keys and takes the heads in turn: the order must not cost what it
+    is there to save.  Bar 5% (two runs of one side differ by 1%)."""
+    H, Hkv, L, rows, D = 32, 8, 32768, 3000, 128
+    q, k, v, kr, vr = make(1, H, Hkv, rows, L, D, torch.bfloat16)
+    pos = torch.arange(L - rows, L, device=DEV)
+    p = make_pattern(L, 64, 0, 8, H)
+    run = lambda a, b: elastic_attention_band(q, a, b, p, 0.1, False, positions=pos)  # noqa: E731
+    shared, repeated = times([lambda: run(k, v), lambda: run(kr, vr)])
+    print(f"  shared {shared * 1e6:.1f} us, repeated {repeated * 1e6:.1f} us", flush=True)
+    assert shared <= 1.05 * repeated
