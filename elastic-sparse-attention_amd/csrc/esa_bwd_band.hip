@@ -1288,31 +1288,65 @@ static void launch_band_dkdv_elem(const BwdArgs& a, int head_dim, dim3 grid, int
 }
 
 // Waves per key block.  One wave takes a block's whole walk, groups * w steps
-// of 32 rows on average and about ln(kv_len / 16) times that for the first
-// blocks of the last layer (interpolation weight 1), so a grid of few rounds of
-// resident waves (2048 at D = 128, 3072 at D = 64: R rounds) lasts as long as
-// its longest walk.  Two to eight waves share a block there; with more rounds
-// one wave a block is faster (no sums handed over, each head's ranges searched
-// once).  Whole band backward, one wave against the rule's count:
-//   weight 1: H=32/4 L=8192 D=128 (R = 1) 3109 -> 1389 us with 8, H=8/2 L=4096
-//   (R = 0.25) 902 -> 283 with 8, H=8/4 L=8192 (R = 1) 742 -> 412 with 4, B=2
-//   H=8/2 L=16384 (R = 2) 1995 -> 1427 with 4, H=8 L=16384 (R = 4) 722 -> 539
-//   with 2; at R = 6.1 within 1%, at R = 8 and 8 kv heads two waves 8% slower;
-//   weight 4/7: H=8/2 L=4096 367 -> 180 with 4, H=32/4 L=8192 1217 -> 1100, H=4
-//   L=4096 (R = 0.5) 136 -> 119 with 2, H=16/8 L=32768 D=64 (R = 5.3) 1128 ->
-//   1084 with 2; one head a kv head at R = 2 .. 2.7 1-5% slower with 2;
-//   weight 0: H=8/2 L=4096 44 -> 38 with 2; at R = 1 5% slower.
+// of 32 rows on average; the walks of a head's low blocks are longer, by
+// ln(1 / (1 - weight)) / weight at interpolation weight < 1 (`over`, less one)
+// and by about ln(kv_len / 16) at the last layer.  A grid of few rounds of
+// resident waves (2048 at D = 128, 3072 at D = 64: R rounds) does not fill the
+// chip or ends in long walks that started late: two to eight waves share a
+// block there.  Sharing costs the sums handed over, each head's ranges searched
+// once per wave, and the neighbouring blocks' common order in L2, so elsewhere
+// one wave a block is faster, 2-15% with a kv head's blocks in XCD order.
+// What decides, of 5800 shapes (groups 1 .. 8, B * Hkv 1 .. 32, D 64 and 128,
+// w 32 .. 64, weights 1/23 .. 1, R 0.2 .. 6; whole band backward, one wave
+// against several):
+//   R <= 0.3 with 4 waves 1.05 .. 2.5x; R <= 0.5 (0.9 with 4 or more query
+//   heads a kv head, 4 waves) 1.0 .. 2.2x;
+//   beyond, `tail`, the rounds of the kv head that runs last (a multiple of 8
+//   kv heads has n / 8 after each other on an XCD, others all n), against
+//   `over`: with whole heads on the XCDs or two heads, H=16/8 L=8192 D=128
+//   weight 22/23 1.12x at tail 2, 0.95 at 3.3, weight 6/7 (w = 32) 1.24 at 1,
+//   0.91 at 3.3; heads spread over the XCDs gain further, H=8/4 L=48k weight
+//   4/7 1.12 at tail 1.5, weight 1/7 0.96; one head less, H=2/1 L=62167 weight
+//   6/23 0.97 at 1.9;
+//   a grid that just starts its second round, 1 < R <= 1.6, 0.98 .. 1.3x but
+//   with one head (0.94);
+//   rounds 3 .. 4 at D = 64, where one wave's walks start unrotated, 0.97 at
+//   tail > 0.8;
+//   weight 1: up to 3.9x at R < 1; 4 waves to 1.8x at R = 2 and 1.5x at 3 .. 4,
+//   2 waves 1.0 .. 1.3x to R = 6, but few heads of one query head each at R in
+//   (3, 4] 0.89 .. 1.04 (H=2 L=63892 627 -> 679 us).
+// By this rule 1% of the shapes whose kernel choice is this kernel are more
+// than 0.5% slower than with one wave (18% by R alone, a limit of 4 rounds for 4
+// query heads and 6 for 2), and the mean of all gains 1.109x (1.103x).
 static int band_dkdv_waves(const BwdArgs& a, int head_dim) {
   const int resident = head_dim == 128 ? 2048 : 3072;
   const float R = (float)a.n_kblk / (float)resident;
-  if (a.pc.a == 0.0f) return R <= 0.5f ? 2 : 1;
-  if (a.pc.a == 1.0f) {
+  const int n = a.B * a.Hkv;
+  const float weight = a.pc.a;
+  if (weight == 0.0f) return R <= 0.5f && a.groups >= 2 ? 2 : 1;
+  if (weight == 1.0f) {
     if (R <= 1.0f) return R <= 0.3f || a.groups >= 4 ? 8 : 4;
+    if (a.groups < 4 && n <= 4 && R > 2.0f && R <= 4.0f) {
+      if (R > (n == 1 ? 2.5f : a.groups == 1 ? 3.0f : 4.0f)) return 1;
+      if (n <= 2 && a.groups > 1) return 2;
+    }
     return R < 4.0f ? 4 : R < 6.0f ? 2 : 1;
   }
-  if (a.groups >= 4) return R < 4.0f ? 4 : 1;
-  if (R <= 1.0f) return R <= 0.3f ? 4 : 2;
-  return a.groups >= 2 && R < 6.0f ? 2 : 1;
+  if (R <= 0.3f) return 4;
+  const int several = a.groups >= 4 ? 4 : 2;
+  const float over = -logf(1.0f - weight) / weight - 1.0f;
+  if (a.groups == 1) return R <= fminf(1.0f, 0.42f + 0.8f * over) ? several : 1;
+  if (R <= (a.groups >= 4 ? 0.9f : 0.5f)) return several;
+  if (n == 1) return R <= 0.55f + 0.5f * over ? several : 1;
+  if (R > (a.groups >= 4 ? 4.0f : 6.0f)) return 1;
+  if (R > 1.0f && R <= 1.6f) return several;
+  const bool whole = n % 8 == 0;
+  const float tail = R / (float)(whole ? n / 8 : n);
+  if (whole || n == 2)
+    return tail <= 0.5f + (n == 2 && a.groups >= 4 ? 1.1f : 0.7f) * over ? several : 1;
+  if (head_dim == 64 && a.groups < 4 && R > 3.0f && R <= 4.0f && tail > 0.8f && over < 1.0f)
+    return 1;
+  return tail <= 5.0f * over ? several : 1;
 }
 
 hipError_t launch_band_dkdv(const BwdArgs& a, int head_dim, const float* lse2,

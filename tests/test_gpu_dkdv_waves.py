@@ -8,6 +8,8 @@ same 16 bits and sum in float32.  Bar: each of a gradient's products carries
 two roundings of 2^-9 (bf16; 2^-12 in f16) and the stored gradients one more
 each; independent over the >= 64 products of a key, at most 4 2^-9 of the
 largest gradient: 8e-3 and 1e-3."""
+import time
+
 import pytest
 import torch
 
@@ -42,3 +44,33 @@ def test_matches_block_sparse(B, H, Hkv, L, D, layer, dtype):
         assert err <= BAR[dtype]
     again = run("band")
     assert all(torch.equal(a, b) for a, b in zip(got, again))
+
+
+def test_shorter_call_is_not_slower():
+    """The rule's several waves a block must not cost time where they are taken:
+    with whole kv heads on the XCDs a grid of 5.9 rounds of resident waves
+    against one of 6.03 at the same pattern, where one wave takes a block.  Two
+    waves made the shorter call 15% slower; with one it is 2% faster (bar 4%,
+    two runs of one side differ by 1%)."""
+    H, Hkv, D = 16, 8, 128
+    calls = []
+    for L in (24161, 24700):
+        g = torch.Generator(device=DEV).manual_seed(L)
+        q, k, v = (torch.randn(1, h, L, D, generator=g, device=DEV, dtype=torch.bfloat16)
+                   for h in (H, Hkv, Hkv))
+        lay = ElasticSparseAttention(6, 8, H, D, 32, L, num_key_value_heads=Hkv).layout(DEV)
+        o, lse = elastic_attention_fwd(q, k, v, lay, 0.1)
+        calls.append(lambda a=(q, k, v, o, lse, torch.randn_like(o), lay, 0.1):
+                     elastic_attention_bwd(*a, dq_kernel="band", dkdv_kernel="band"))
+    best = [float("inf")] * 2
+    for _ in range(8):
+        for i, f in enumerate(calls):
+            f()
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(8):
+                f()
+            torch.cuda.synchronize()
+            best[i] = min(best[i], (time.perf_counter() - t0) / 8)
+    print(f"  {best[0] * 1e6:.0f} us, longer {best[1] * 1e6:.0f} us", flush=True)
+    assert best[0] <= 1.04 * best[1]
