@@ -1007,10 +1007,23 @@ __global__ __launch_bounds__(64 * S, 2) void band_dkdv_kernel(BwdArgs A, const f
       }
     };
 
-    __amdgpu_buffer_rsrc_t qrs, ors, srs;
+    if constexpr (WIN) h = kvh * A.groups + p_first / (win_steps * ROWS);
     // head h's Q and dO rows; its delta row and, lse_off bytes further, its
-    // lse2 row
-    auto set_head = [&](int h) {
+    // lse2 row.  Initialised here, and assigned only for WIN's next head: with
+    // one lambda that assigns both, the dilated forms' step loop is scheduled
+    // differently and H=32 L=8192 D=128 took 0.3-0.4% longer (1270 against 1265
+    // us, three runs).
+    __amdgpu_buffer_rsrc_t qrs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(A.q + (int64_t)b * A.qsb + (int64_t)h * A.qsh), (short)0, A.q_len * qss2,
+        0x00020000);
+    __amdgpu_buffer_rsrc_t ors = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(A.dout + (int64_t)b * A.dosb + (int64_t)h * A.dosh), (short)0, A.q_len * oss2,
+        0x00020000);
+    __amdgpu_buffer_rsrc_t srs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(A.delta + ((int64_t)b * A.H + h) * A.qpad), (short)0, lse_off + 4 * A.qpad,
+        0x00020000);
+    auto next_head = [&] {
+      ++h;
       qrs = __builtin_amdgcn_make_buffer_rsrc(
           (void*)(A.q + (int64_t)b * A.qsb + (int64_t)h * A.qsh), (short)0, A.q_len * qss2,
           0x00020000);
@@ -1021,8 +1034,6 @@ __global__ __launch_bounds__(64 * S, 2) void band_dkdv_kernel(BwdArgs A, const f
           (void*)(A.delta + ((int64_t)b * A.H + h) * A.qpad), (short)0, lse_off + 4 * A.qpad,
           0x00020000);
     };
-    if constexpr (WIN) h = kvh * A.groups + p_first / (win_steps * ROWS);
-    set_head(h);
     // Q or dO rows of the step whose slot rows hold `row` -> slot dst (after
     // the step's reads of dst)
     auto issue_rows = [&](__amdgpu_buffer_rsrc_t rs, int ss2, int row, lds_u16* dst) {
@@ -1062,7 +1073,7 @@ __global__ __launch_bounds__(64 * S, 2) void band_dkdv_kernel(BwdArgs A, const f
         map_step(P + ROWS, e, row_n, ent_n);
         if constexpr (WIN) {
           const int hn = kvh * A.groups + (P + ROWS) / (win_steps * ROWS);
-          if (hn != h) set_head(h = hn);
+          if (hn != h) next_head();
         }
       }
       // the key of slot row (lane % 32), -1 when masked or empty
