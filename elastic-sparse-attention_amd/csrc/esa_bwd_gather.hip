@@ -230,9 +230,11 @@ __global__ __launch_bounds__(256) void bwd_kv_kernel(GatherBwdArgs A) {
 // float32 B=2 H=8 L=4096 D=64 467 -> 91 and 564 -> 106 us; bf16 D=96 H=16/4
 // L=5001 496 -> 130 and 1036 -> 226 us.
 
-// One wave per (batch, head, query row): dQ and the row's (lse, delta).  A
-// chunk's K and V rows are all in flight before the first score, K stays in registers for dQ, and each lane forms one entry's dS.
-// Bound by the L2 row gathers (2 w rows a query row).
+// One wave per (batch, head, query row): dQ and the row's (lse, delta).  The
+// list is walked in chunks of NMAX load instructions of K and as many of V
+// (bwd_in_flight), all of a chunk's in flight before its first score; K stays
+// in registers for dQ, and each lane forms one entry's dS.  Bound by the L2 row
+// gathers (2 w rows a query row).
 template <Elem E, int LPK, bool PATTERN>
 __global__ __launch_bounds__(256, 2) void rows_coop_kernel(GatherBwdArgs A) {
   using T = typename ElemT<E>::T;
@@ -554,7 +556,6 @@ unsigned grid_for(int64_t n) {
 // of both passes: 125 -> 60 us against one-pair-at-a-time stores and separate
 // key and chunked-scan launches (first scatter 52 -> 16 us); 5.1M: 230 -> 105.
 constexpr int kSortTile = 4096;
-constexpr int kScanChunk = 2048;  // of the workspace's size formula
 
 // Sort keys of every entry (batch-independent): kv_head * kv_len + key of a
 // valid entry with a key in [0, kv_len), else the sentinel Hkv * kv_len; and
@@ -878,11 +879,7 @@ hipError_t launch_elem(const GatherBwdArgs& a0, bool pattern, hipStream_t stream
 
 }  // namespace
 
-void gather_bwd_sort_sizes(int64_t n, int64_t* hist_ints, int64_t* part_ints) {
-  const int64_t nb = (n + kSortTile - 1) / kSortTile;
-  *hist_ints = 256 * nb;
-  *part_ints = (256 * nb + kScanChunk - 1) / kScanChunk;
-}
+int64_t gather_bwd_hist_ints(int64_t n) { return 256 * ((n + kSortTile - 1) / kSortTile); }
 
 hipError_t launch_gather_bwd(const GatherBwdArgs& a, bool pattern, hipStream_t stream) {
   if (a.B <= 0 || a.H <= 0 || a.kv_len <= 0) return hipSuccess;

@@ -173,9 +173,10 @@ void plan_xcd_grid(const int32_t* row_ptr, int nqb, int nq, int batch, int H,
 esa_status hip_status(hipError_t e) { return e == hipSuccess ? ESA_OK : ESA_ERR_HIP; }
 
 // Byte offsets of the gather backward's workspace regions (each 256-byte
-// aligned): per batch element and entry a dV and a dK coefficient, two
-// (key, entry id) pair buffers for the sort, the per-key segment starts and
-// the sort's digit histograms and their scan.
+// aligned): two float32 words per batch element and entry (a dV and a dK
+// coefficient, or the cooperative-row kernels' space, GatherBwdArgs), two (key,
+// entry id) pair buffers for the sort, the per-key segment starts and the
+// sort's digit histograms and their scan.
 struct GatherBwdLayout {
   int64_t E;  // entries per batch element: H * q_len * w
   size_t cp, cs, ka, va, kb, vb, seg, hist, offs, total;
@@ -189,8 +190,10 @@ esa_status gather_bwd_layout(const esa_bwd_args* a, int32_t w, GatherBwdLayout* 
   // entry ids and sorted positions are 32-bit; the sort keys' sentinel is
   // Hkv * kv_len
   if (E >= INT32_MAX || (int64_t)a->num_kv_heads * a->kv_len >= INT32_MAX) return ESA_ERR_SHAPE;
-  int64_t hist_ints = 0, part_ints = 0;
-  gather_bwd_sort_sizes(E, &hist_ints, &part_ints);
+  const int64_t hist_ints = gather_bwd_hist_ints(E);
+  // not read: one int32 per 2048 histogram entries, which the documented
+  // workspace size has always counted
+  const int64_t unused_ints = (hist_ints + 2047) / 2048;
   auto up = [](size_t x) { return (x + 255) / 256 * 256; };
   size_t at = 0;
   auto take = [&](size_t bytes) {
@@ -208,7 +211,7 @@ esa_status gather_bwd_layout(const esa_bwd_args* a, int32_t w, GatherBwdLayout* 
   L->seg = take(((size_t)a->num_kv_heads * a->kv_len + 1) * 4);
   L->hist = take((size_t)hist_ints * 4);
   L->offs = take((size_t)hist_ints * 4);
-  take((size_t)part_ints * 4);  // spare: the size that callers allocate stays the same
+  take((size_t)unused_ints * 4);
   L->total = at;
   return ESA_OK;
 }

@@ -158,8 +158,9 @@ struct GatherArgs {
 };
 
 // Arguments of the gather backward (any index source, float32 / bfloat16 /
-// float16): per-row pass (dQ and each entry's dK / dV coefficients), a stable
-// sort of the (kv head, key) of every valid entry, then a key-major pass.
+// float16): per-row pass (dQ, and each entry's dK / dV coefficients or, in the
+// cooperative-row form, the row's (lse, delta)), a stable sort of the (kv head,
+// key) of every valid entry, then a key-major pass.
 struct GatherBwdArgs {
   const void* q;
   const void* k;
@@ -185,8 +186,11 @@ struct GatherBwdArgs {
   IndexSource src;
   DropoutArgs drop;
   int64_t E;          // entries per batch element: H * q_len * w
-  float* cp;          // [B][E] dV coefficient of each entry (dropout-scaled p)
-  float* cs;          // [B][E] dK coefficient of each entry (sm_scale * dS)
+  // per-lane kernels: [B][E] dV coefficient of each entry (dropout-scaled p)
+  // and dK coefficient (sm_scale * dS); the cooperative-row kernels form both
+  // again and keep ld2 and partial in the 2 B E floats from cp on
+  float* cp;
+  float* cs;
   uint32_t* keys_in;  // [E] kv_head * kv_len + key of a valid in-range entry, else the sentinel
   uint32_t* vals_in;  // [E] entry ids
   uint32_t* keys_out;
@@ -197,8 +201,8 @@ struct GatherBwdArgs {
   int key_bits;       // bits of the sort keys
   // the cooperative-row kernels (set by the launcher): (lse, delta) of each
   // row [B][H q_len] and partial sums [B][n_windows][2][2][D] of long
-  // segments, both in cp / cs's space; bytes spanned by a head's K / V rows and
-  // a batch element's q / dO rows; blocks per XCD range; divisors w and q_len
+  // segments; bytes spanned by a head's K / V rows and a batch element's q / dO
+  // rows; blocks per XCD range; divisors w and q_len
   float2* ld2;
   float* partial;
   int part, n_windows;
@@ -310,9 +314,8 @@ hipError_t launch_band_dkdv(const BwdArgs& a, int head_dim, const float* lse2,
                             hipStream_t stream);
 hipError_t launch_gather_fwd(const GatherArgs& a, bool pattern, hipStream_t stream);
 hipError_t launch_gather_weights(const GatherArgs& a, bool pattern, hipStream_t stream);
-// int32 entries of the sort's digit histograms (and of their scan), and a
-// spare region's (one per 2048 of them), for n pairs
-void gather_bwd_sort_sizes(int64_t n, int64_t* hist_ints, int64_t* part_ints);
+// int32 entries of the sort's digit histograms (and of their scan) for n pairs
+int64_t gather_bwd_hist_ints(int64_t n);
 hipError_t launch_gather_bwd(const GatherBwdArgs& a, bool pattern, hipStream_t stream);
 hipError_t launch_tile_masks(const PatternConsts& pc, const int32_t* row_ptr, const int32_t* col_idx,
                              int nqb, int q_len, uint32_t* mask_t, hipStream_t stream);

@@ -422,8 +422,8 @@ esa_status esa_elastic_bwd(const esa_bwd_args* a, const esa_pattern* p,
  * need for index lists of attn_length entries per row: per batch element and
  * entry two float32 words (coefficients, or the rows' lse and delta and partial
  * sums), four uint32 arrays of entries for the sort,
- * (num_kv_heads * kv_len + 1) int32 segment starts, and the sort's
- * histograms (each region 256-byte aligned).  Requires num_heads * q_len *
+ * (num_kv_heads * kv_len + 1) int32 segment starts, the sort's histograms and
+ * one unused int32 per 2048 of their entries (each region 256-byte aligned).  Requires num_heads * q_len *
  * attn_length and num_kv_heads * kv_len below 2^31 - 1. */
 esa_status esa_gather_bwd_workspace_size(const esa_bwd_args* a, int32_t attn_length,
                                          size_t* workspace_bytes);
