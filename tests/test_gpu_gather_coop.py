@@ -100,9 +100,9 @@ def test_keys_that_every_row_lists(dtype, D, L):
 @pytest.mark.parametrize("dtype,D", [(torch.float32, 64), (torch.bfloat16, 80)])
 @pytest.mark.parametrize("dropout_p", [0.0, 0.3])
 def test_unaligned_rows_agree(dtype, D, dropout_p, monkeypatch):
-    """Rows 4 elements off 16 bytes take the per-lane kernels; both forms
-    give the same gradients to float32 summation order, also with dropout (the
-    same keep decisions)."""
+    """A q one element off 16 bytes takes the per-lane kernels (coop_applies
+    wants every tensor aligned); both forms give the same gradients to float32
+    summation order, also with dropout (the same keep decisions)."""
     B, H, Hkv, L = 2, 4, 2, 700
     pat = make_pattern(L, 64, 7, 8, H)
     q, k, v, go, _ = inputs(B, H, Hkv, L, D, dtype, 3)
@@ -117,3 +117,56 @@ def test_unaligned_rows_agree(dtype, D, dropout_p, monkeypatch):
     got = elastic_attention_bwd_rows(off, *d[1:], o, lse, go.to(DEV), pat, 0.1,
                                      dropout_p=dropout_p, seed=9)
     check(got, [t.double().cpu() for t in want], dtype)
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 80), (torch.float16, 64)])
+def test_rows_four_elements_off(dtype, D, monkeypatch):
+    """q, k, v and dO 4 elements (8 bytes) off 16 bytes: as given they take the
+    per-lane kernels; by default they are copied to aligned rows first, and the
+    gradients are the aligned call's bit for bit."""
+    B, H, Hkv, L = 2, 4, 2, 300
+    pat = make_pattern(L, 48, 5, 8, H)
+    q, k, v, go, _ = inputs(B, H, Hkv, L, D, dtype, 4)
+    d = [t.to(DEV) for t in (q, k, v, go.transpose(1, 2).contiguous())]
+
+    def off(t):
+        r = torch.empty(t.numel() + 4, dtype=dtype, device=DEV)[4:].view(t.shape)
+        assert r.data_ptr() % 16 == 8
+        return r.copy_(t)
+
+    o, lse = elastic_attention_rows(*d[:3], pat, 0.1)
+    want = elastic_attention_bwd_rows(*d[:3], o, lse, d[3], pat, 0.1)
+    e = [off(t) for t in d]
+    copied = elastic_attention_bwd_rows(*e[:3], o, lse, e[3], pat, 0.1)
+    assert all(torch.equal(a, b) for a, b in zip(copied, want))
+    monkeypatch.setattr(esa, "_row_align", lambda t: 4)
+    check(elastic_attention_bwd_rows(*e[:3], o, lse, e[3], pat, 0.1),
+          [t.double().cpu() for t in want], dtype)
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 64), (torch.float32, 132),
+                                     (torch.bfloat16, 96), (torch.float16, 256)])
+def test_strided_rows(dtype, D):
+    """q, k, v and dO as transposed views of [B, L, heads, D], as a projection
+    writes them, and K and V as the first rows of a longer cache: the contiguous
+    call's gradients bit for bit (the same kernels, only other strides)."""
+    B, H, Hkv, L = 2, 6, 2, 333
+    pat = make_pattern(L, 64, 6, 8, H)
+    q, k, v, go, g = inputs(B, H, Hkv, L, D, dtype, 5)
+    d = [t.to(DEV) for t in (q, k, v)]
+    dout = go.transpose(1, 2).contiguous().to(DEV)
+    o, lse = elastic_attention_rows(*d, pat, 0.1)
+    want = elastic_attention_bwd_rows(*d, o, lse, dout, pat, 0.1)
+    s = [t.transpose(1, 2).contiguous().transpose(1, 2) for t in d]
+    assert not s[0].is_contiguous()
+    o1, lse1 = elastic_attention_rows(*s, pat, 0.1)
+    assert torch.equal(o1, o) and torch.equal(lse1, lse)
+    # dO of [B, H, L, D] storage, passed as [B, L, H, D]
+    got = elastic_attention_bwd_rows(*s, o, lse, go.to(DEV).transpose(1, 2), pat, 0.1)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    cache = [torch.randn(B, Hkv, L + 50, D, generator=g).to(dtype).to(DEV) for _ in range(2)]
+    for c, t in zip(cache, d[1:]):
+        c[:, :, :L] = t
+    got = elastic_attention_bwd_rows(d[0], cache[0][:, :, :L], cache[1][:, :, :L], o, lse, dout,
+                                     pat, 0.1)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
