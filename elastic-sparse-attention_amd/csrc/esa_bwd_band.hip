@@ -1329,6 +1329,9 @@ static void launch_band_dkdv_elem(const BwdArgs& a, int head_dim, dim3 grid, int
 // By this rule 1% of the shapes whose kernel choice is this kernel are more
 // than 0.5% slower than with one wave (18% by R alone, a limit of 4 rounds for 4
 // query heads and 6 for 2), and the mean of all gains 1.109x (1.103x).
+// (The caller that picks the kernel by staged blocks per row group alone still
+// takes the block-sparse dK/dV at many of the smallest of these grids, and
+// few of the gains at R < 0.5 are reached by default.)
 static int band_dkdv_waves(const BwdArgs& a, int head_dim) {
   const int resident = head_dim == 128 ? 2048 : 3072;
   const float R = (float)a.n_kblk / (float)resident;

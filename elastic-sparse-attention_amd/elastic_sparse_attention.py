@@ -498,6 +498,15 @@ MFMA_DTYPES = (torch.bfloat16, torch.float16)
 # switch between 14.4 and 18.7; at D = 64 the tile dQ is faster up to 11.9
 # (within 1% with 8 kv heads), the band dQ from 14.0 (by 3-5%); the tile
 # dK/dV up to 15.5 (by 6-17%), the band dK/dV from 18.7.
+# The dK/dV figures are of one wave per key block and the rule sees neither
+# query heads per kv head nor the grid's rounds.  Where several waves share a
+# block (grids of few rounds, band_dkdv_waves) and kv heads are shared, the
+# band dK/dV is faster below the crossover too, and only dkdv_kernel="band"
+# takes it: whole backward, tile against band dK/dV at layers 1 / 3 / 4 / 7 of
+# 8, L=4096 D=128 H=8/2 130 / 287 / 362 / 587 us against 132 / 174 / 199 / 343,
+# H=8/1 216 / 507 / 644 / 1047 against 182 / 231 / 262 / 481, D=64 H=8/2 95 /
+# 214 / 275 / 399 against 88 / 115 / 129 / 189; without sharing, H=8 66 / 126 /
+# 154 / 240 against 119 / 155 / 170 / 227.
 BAND_CROSSOVER = {128: 18.5, 64: 13.0}
 BWD_DQ_CROSSOVER = {128: 16.5, 64: 13.0}
 BWD_DKDV_CROSSOVER = {128: 16.5, 64: 17.0}
