@@ -24,6 +24,8 @@
 // aligned rows) reads each K and V row with a lane per 16 bytes.
 // gather_weights_kernel writes the naive path's attention weights from the
 // forward's lse.
+#include <algorithm>
+
 #include "esa_gather.hpp"
 
 namespace esa {
@@ -56,16 +58,17 @@ __global__ __launch_bounds__(256) void gather_fwd_kernel(GatherArgs A) {
 // gather_fwd_kernel (accurate expf; only the order of float32 additions
 // differs).  Loads are buffer loads with 32-bit offsets (BUF; a masked entry
 // reads zeros without a fetch) unless a head's K or V spans 2 GiB.
-// XCD x takes a contiguous range of the waves, so its L2 holds the K and V of
-// a few heads: explicit lists bf16 B=2 H=8 L=4096 D=128 200 -> 185 us,
-// float32 D=64 158 -> 151 us, the decode steps unchanged.
+// Where an L2 holds the keys that a head's rows list (xcd_ranges), XCD x takes
+// a contiguous range of the waves, so it reads the K and V of a few heads:
+// explicit lists bf16 B=2 H=8 L=4096 D=128 200 -> 185 us, float32 D=64 158 ->
+// 151 us, the decode steps unchanged.
 template <Elem E, int LPK, int NMAX, bool BUF, bool PATTERN>
 __global__ __launch_bounds__(256, 2) void gather_rows_kernel(GatherArgs A) {
   __shared__ float sc_all[4][64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  // XCD x (blockIdx % 8) takes a contiguous range of rows
-  const int wv = (int)(blockIdx.x & 7) * A.waves_per_xcd + (int)(blockIdx.x >> 3) * 4 + wave;
+  // (in ranges, XCD x = blockIdx % 8 taking a contiguous one, or in turn)
+  const int wv = (int)(blockIdx.x & 7) * A.xcd_step + (int)(blockIdx.x >> 3) * A.block_step + wave;
   if (wv >= A.waves) return;  // whole wave leaves; no block-level barrier below
   const int bh = wv / A.q_len, r = wv % A.q_len;
   const int b = bh / A.H, h = bh % A.H;
@@ -130,6 +133,25 @@ bool rows_aligned16(const GatherArgs& a, int es) {
   return true;
 }
 
+// Whether each XCD takes a contiguous range of the waves, or all of them take
+// every head's rows in turn: by the bytes of K and V that a head's rows list,
+// its window over the keys (interpolation weight x kv_len; half of kv_len for
+// explicit lists) or, for few rows, w keys a row.  Ranges against turns, inputs
+// changing from call to call, float32 and bf16, D 64 .. 256, L 2048 .. 65536: up
+// to 5 MB ranges 1-30% faster (float32 H=8 L=4096 D=128 layer 4 of 8 169 against
+// 183 us; 64 rows of H=32/8 L=32768 11.8 against 18.9); beyond, where a head's
+// keys overflow an XCD's L2, turns 3-64% faster (presumably because eight
+// XCDs then miss the same keys at about the same time; H=8/2 L=32768 D=128 layer
+// 4 1216 -> 992 us, H=2/1 L=65536 712 -> 658); at weight 1 past 32 MB, with
+// hardly a key shared, ranges 3-13% faster again.
+bool xcd_ranges(const GatherArgs& a, int es, bool pattern) {
+  const double weight = pattern ? (double)a.src.pc.a : 0.5;
+  const double window = std::max(weight * a.kv_len, (double)a.src.w);
+  const double keys = std::min(window, (double)a.q_len * a.src.w);
+  const double bytes = 2.0 * keys * a.D * es;
+  return bytes <= 5e6 || (pattern && a.src.pc.a == 1.0f && bytes > 32e6);
+}
+
 template <Elem E, int LPK, int NMAX, bool BUF>
 void launch_rows(const GatherArgs& a, unsigned blocks, bool pattern, hipStream_t stream) {
   if (pattern)
@@ -162,7 +184,9 @@ void launch_gather_elem(const GatherArgs& a, bool pattern, hipStream_t stream) {
   if (rows_aligned16(a, ElemT<E>::kBytes) && per_xcd * 8 * 256 <= (int64_t)UINT32_MAX) {
     GatherArgs c = a;
     c.waves = (int)waves;  // (< 2^26: the test above)
-    c.waves_per_xcd = (int)per_xcd * 4;
+    const bool ranges = xcd_ranges(a, ElemT<E>::kBytes, pattern);
+    c.xcd_step = ranges ? (int)per_xcd * 4 : 4;
+    c.block_step = ranges ? 4 : 32;
     const int64_t ks = row_span(a.kv_len, a.kss, 1, 0, a.D, ElemT<E>::kBytes);
     const int64_t vs = row_span(a.kv_len, a.vss, 1, 0, a.D, ElemT<E>::kBytes);
     const bool buf = ks < kMaxSpan && vs < kMaxSpan;

@@ -152,9 +152,10 @@ struct GatherArgs {
   void* weights;
   int64_t wsb, wsh, wss;
   // the cooperative kernel (set by the launcher): bytes a head's K / V rows
-  // span; waves, and waves per XCD range
+  // span; waves, and the first wave's step from an XCD's range to the next's
+  // and from one of an XCD's blocks to its next
   int k_span, v_span;
-  int waves, waves_per_xcd;
+  int waves, xcd_step, block_step;
 };
 
 // Arguments of the gather backward (any index source, float32 / bfloat16 /

@@ -12,6 +12,8 @@ p, and with it the gradients, carry that error as a relative one.  bfloat16 and
 float16: one rounding of the stored gradient, 2^-8 and 2^-11, plus the same
 sums: 6e-3 and 1e-3.
 """
+import time
+
 import pytest
 import torch
 
@@ -170,3 +172,50 @@ def test_strided_rows(dtype, D):
     got = elastic_attention_bwd_rows(d[0], cache[0][:, :, :L], cache[1][:, :, :L], o, lse, dout,
                                      pat, 0.1)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("dtype,H,Hkv,L,D,layer", [
+    (torch.float32, 2, 1, 9001, 128, 4),   # 5.3 MB of keys a head: rows in turn
+    (torch.float32, 3, 1, 8003, 128, 4),   # 4.7 MB: a range an XCD
+    (torch.float32, 2, 2, 5001, 64, 7),    # weight 1
+    (torch.bfloat16, 5, 1, 12001, 160, 6)])
+def test_row_orders(dtype, H, Hkv, L, D, layer):
+    """The order in which the XCDs take the rows (in ranges or in turn, by the
+    keys a head's rows list) leaves no row out: the whole call against the same
+    rows at 150 positions, whose few keys take ranges.  The two take chunks of
+    different lengths: float32 sums, and one rounding to bf16."""
+    g = torch.Generator(device=DEV).manual_seed(L)
+    q, k, v = (torch.randn(1, h, L, D, generator=g, device=DEV, dtype=dtype)
+               for h in (H, Hkv, Hkv))
+    p = make_pattern(L, 64, layer, 8, H)
+    o, lse = elastic_attention_rows(q, k, v, p, 0.1)
+    pos = torch.randperm(L, generator=g, device=DEV)[:150]
+    pos[:3] = torch.tensor([0, L - 1, L - 2], device=DEV)
+    o1, lse1 = elastic_attention_rows(q[:, :, pos].contiguous(), k, v, p, 0.1, positions=pos)
+    bar = 2e-6 if dtype == torch.float32 else 2.0 ** -8
+    assert (lse[:, :, pos] - lse1).abs().max() <= 2e-6 * lse.abs().max()
+    assert (o[:, pos].float() - o1.float()).abs().max() <= bar * o.abs().max().item()
+    assert torch.isfinite(o.float()).all()
+
+
+def test_long_rows_by_window():
+    """Rows whose keys exceed an XCD's L2: layer 4's rows list keys of the last
+    four sevenths of what layer 7's do and take no longer (an order that keeps a
+    head on one XCD made them 10% slower; bar 3%)."""
+    H, L, D = 8, 32768, 128
+    g = torch.Generator(device=DEV).manual_seed(1)
+    sets = [tuple(torch.randn(1, h, L, D, generator=g, device=DEV) for h in (H, 2, 2))
+            for _ in range(2)]
+    best = [float("inf")] * 2
+    for _ in range(6):
+        for i, layer in enumerate((4, 7)):
+            p = make_pattern(L, 64, layer, 8, H)
+            elastic_attention_rows(*sets[0], p, 0.1)
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            for n in range(8):
+                elastic_attention_rows(*sets[n % 2], p, 0.1)
+            torch.cuda.synchronize()
+            best[i] = min(best[i], (time.perf_counter() - t0) / 8)
+    print(f"  layer 4 {best[0] * 1e6:.0f} us, layer 7 {best[1] * 1e6:.0f} us", flush=True)
+    assert best[0] <= 1.03 * best[1]
